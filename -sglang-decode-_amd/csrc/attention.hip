@@ -5,10 +5,7 @@
 
 namespace sgd {
 int launch_attention_generic(const sgd_decode_args &a, bool vec, hipStream_t stream);
-int launch_attention_valu(const sgd_decode_args &a, hipStream_t stream);
-int launch_attention_mfma(const sgd_decode_args &a, hipStream_t stream);
-bool valu_supported(const sgd_decode_args &a);
-bool mfma_supported(const sgd_decode_args &a);
+int launch_attention_pipe(const sgd_decode_args &a, hipStream_t stream);
 }
 
 using namespace sgd;
@@ -24,6 +21,13 @@ bool vector_layout(const sgd_decode_args &a) {
     for (int i = 0; i < 3; ++i)
         if (a.k_stride[i] % 8 != 0 || a.v_stride[i] % 8 != 0) return false;
     return true;
+}
+
+// The pipelined kernel: groups up to 16 (the MFMA's N), those layouts, and page strides that
+// keep a 32-bit index times the stride a valid 64-bit byte offset.
+bool pipe_supported(const sgd_decode_args &a, int max_group) {
+    const int g = a.query_heads / a.kv_heads;
+    return g <= max_group && vector_layout(a) && a.k_stride[0] < (1ll << 40) && a.v_stride[0] < (1ll << 40);
 }
 
 }  // namespace
@@ -56,23 +60,22 @@ int check_args(const sgd_decode_args *args) {
 int resolve_kernel(const sgd_decode_args &a) {
     switch (a.kernel) {
         case SGD_KERNEL_AUTO:
-            // The VALU kernel for groups <= 4 (1-2% faster than the MFMA kernel, whose 16
-            // MFMA columns are then three-quarters padding, on the Llama-3-8B layers
-            // measured), else the MFMA one (groups up to 16), else the generic kernel.
-            // All three merge a task's wave states in a fixed order, so a launch is
-            // bitwise repeatable whatever the worker count.
-            if (valu_supported(a)) return SGD_KERNEL_VALU;
-            if (mfma_supported(a)) return SGD_KERNEL_MFMA;
+            // One kernel serves every group (the two names keep the groups they were asked
+            // for under); layouts it does not take go to the generic one.  Both merge a task's
+            // wave states in a fixed order, so a launch is bitwise repeatable whatever the
+            // worker count.
+            if (pipe_supported(a, 4)) return SGD_KERNEL_VALU;
+            if (pipe_supported(a, 16)) return SGD_KERNEL_MFMA;
             return SGD_KERNEL_GENERIC;
         case SGD_KERNEL_GENERIC:
             return SGD_KERNEL_GENERIC;
         case SGD_KERNEL_VALU:
-            if (!valu_supported(a))
+            if (!pipe_supported(a, 4))
                 return einval("persistent_decode: the VALU kernel needs group <= 4, head_dim 64/128/256, unit dim "
                               "stride and 16-byte aligned rows");
             return SGD_KERNEL_VALU;
         case SGD_KERNEL_MFMA:
-            if (!mfma_supported(a))
+            if (!pipe_supported(a, 16))
                 return einval("persistent_decode: the MFMA kernel needs group <= 16, head_dim 64/128/256, unit dim "
                               "stride and 16-byte aligned rows");
             return SGD_KERNEL_MFMA;
@@ -96,9 +99,8 @@ extern "C" int sgd_persistent_decode(const sgd_decode_args *args, void *stream) 
     clear_stale_error();
     switch (kernel) {
         case SGD_KERNEL_VALU:
-            return launch_attention_valu(a, (hipStream_t)stream);
         case SGD_KERNEL_MFMA:
-            return launch_attention_mfma(a, (hipStream_t)stream);
+            return launch_attention_pipe(a, (hipStream_t)stream);
         default:
             return launch_attention_generic(a, vector_layout(a), (hipStream_t)stream);
     }

@@ -1,4 +1,5 @@
-// Wave64 building blocks shared by the VALU decode-attention kernels: packed
+// Wave64 building blocks of the VALU split-KV decode (and DPP and 16-bit packing helpers of
+// the pipelined kernel): packed
 // 16-bit dot products, DPP cross-lane moves, the paged/CSR row gather of one tile,
 // and the tile's QK^T / online-softmax / P.V math, for head_dim D in {64, 128, 256}.
 //

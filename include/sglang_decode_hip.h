@@ -37,8 +37,10 @@ enum sgd_dtype { SGD_BF16 = 0, SGD_FP16 = 1 };
 enum sgd_kernel {
     SGD_KERNEL_AUTO = 0,     /* pick by geometry (see sgd_persistent_decode) */
     SGD_KERNEL_GENERIC = 1,  /* any strides/alignment, any supported geometry */
-    SGD_KERNEL_VALU = 2,     /* per-task VALU kernel: LDS-staged K/V tiles, DPP reductions, dot2 (group <= 4) */
-    SGD_KERNEL_MFMA = 3      /* MFMA QK^T and PV, K/V straight from HBM into operands (group <= 16) */
+    /* Groups <= 4 and <= 16 of one pipelined MFMA kernel (unit dim stride, 16-byte aligned rows); both
+     * names are kept, and refuse what they refused when they named kernels of their own. */
+    SGD_KERNEL_VALU = 2,
+    SGD_KERNEL_MFMA = 3
 };
 
 /* Human-readable description of the last SGD_EINVAL / launch failure (thread-local). */
