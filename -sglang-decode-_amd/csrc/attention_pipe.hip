@@ -24,7 +24,7 @@
 // Measured (us per launch, captured graph; before = a VALU kernel for groups <= 4 and a separate MFMA
 // kernel with 64 B row pieces): 8B-class heads, 64 requests, 395 MB 74.3 -> 72; 70B-class heads, 32
 // requests in 16-token pages, 1.14 GB 193 -> 186; 32 kv heads, no grouping, 537 MB 103 -> 95; head_dim 64
-// 58.9 -> 51.5; head_dim 256 82.5 -> 78; one request of 8k tokens 18.1 -> 15.6; one kv head of 8 query heads,
+// 58.9 -> 51.5; head_dim 256 82.5 -> 78; one request of 8k tokens 18.1 -> 12.8 (15.6 with every worker counted); one kv head of 8 query heads,
 // 64 requests 24.5 -> 21.1.
 //
 // Lane l of a compute wave is (m, j) = (l % 16, l / 16).  MFMA operands of 16x16xK:
@@ -570,8 +570,9 @@ __device__ __forceinline__ void helper_wave(const sgd_decode_args &a, PipeShared
         wave0_tiles += n0;
     }
     // The last worker to finish puts the claim counter back to zero for the next launch
-    // (relaxed: see for_each_task).
-    if (a.done_counter && lane == 0) {
+    // (relaxed: see for_each_task).  Only schedules that claim move it: without a task, 512
+    // workers' atomics on one word would delay the others' first loads by ~3 us.
+    if (dynamic && a.done_counter && lane == 0) {
         const int32_t done = __hip_atomic_fetch_add(a.done_counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (done == a.workers - 1) {
             __hip_atomic_store(a.counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
