@@ -183,7 +183,7 @@ __device__ __forceinline__ int32_t request_of(const int32_t *offsets, int32_t bc
 // are those of stage_emit_records.
 __device__ void stage_emit_by_record(const RowMirror &rows, int32_t total, int32_t bcap, int32_t *request,
                                      int32_t *split, int32_t *begin, int32_t *end, int32_t *weight,
-                                     int32_t block_kv, int32_t *weight_mirror) {
+                                     int32_t block_kv, int32_t *weight_mirror, int4 *recs) {
     for (int32_t idx = threadIdx.x; idx < total; idx += kPlanThreads) {
         const int32_t r = request_of(rows.offsets, bcap, idx);
         const int32_t s = wadd(idx, -rows.offsets[r]);
@@ -197,13 +197,14 @@ __device__ void stage_emit_by_record(const RowMirror &rows, int32_t total, int32
         const int32_t w = cdiv(wadd(e, -b), block_kv);
         weight[idx] = w;
         weight_mirror[idx] = w;
+        if (recs) recs[idx] = make_int4(r, s, b, e);
     }
 }
 
+// The number of k in 1 .. buckets - 1 with w > 2^(k - 1): ceil(log2 w), capped.
 __device__ __forceinline__ int bucket_of(int32_t w, int buckets) {
-    int b = 0;
-    for (int k = 1; k < buckets; ++k) b += w > (1 << (k - 1));
-    return b;
+    const int b = w <= 1 ? 0 : 32 - __builtin_clz((uint32_t)(w - 1));
+    return min(b, buckets - 1);
 }
 
 // ---------------------------------------------------------------- bucket tables
@@ -211,24 +212,12 @@ struct BucketOf {
     int32_t rbase, pbase, width, pp, pt;
 };
 
-// The bucket holding sorted record position j (buckets are laid out heaviest first),
-// read from the LDS tables at uniform addresses.  The callers loop over tasks, so the
-// lanes past the last task are switched off: a per-lane register copy of the tables read
-// back with v_readlane would read those lanes' stale registers (the compiler loads the
-// copy inside the loop), while an LDS broadcast gives every active lane the table.
-__device__ __forceinline__ BucketOf bucket_at(const PlanShared &sh, int32_t j, int buckets) {
-    BucketOf o{0, 0, 1, 0, 0};
-    for (int q = buckets - 1; q >= 0; --q) {
-        const int32_t lo = sh.bucket_record_base[q], n = sh.bucket_size[q];
-        if (j >= lo && j < lo + n) {
-            o.rbase = lo;
-            o.pbase = sh.bucket_pack_base[q];
-            o.width = sh.bucket_width[q];
-            o.pp = sh.bucket_packed_packs[q];
-            o.pt = sh.bucket_packed_tasks[q];
-        }
-    }
-    return o;
+// Bucket b's tables, read from LDS by every lane for itself.  (A per-lane register copy read
+// back with v_readlane would read the stale registers of lanes past the last task, which the
+// callers' loops switch off.)
+__device__ __forceinline__ BucketOf bucket_tables(const PlanShared &sh, int b) {
+    return BucketOf{sh.bucket_record_base[b], sh.bucket_pack_base[b], sh.bucket_width[b], sh.bucket_packed_packs[b],
+                    sh.bucket_packed_tasks[b]};
 }
 
 // The pack that task `task` starts (its index, and its task count in `count`), or -1
@@ -238,7 +227,8 @@ __device__ __forceinline__ int32_t pack_of(const BucketOf &o, int32_t task, int3
     const int32_t p = task - o.rbase * hkv;
     if (p < o.pt) {
         count = o.width;
-        return p % o.width == 0 ? o.pbase + p / o.width : -1;
+        const int32_t u = (int32_t)((uint32_t)p / (uint32_t)o.width);
+        return p == u * o.width ? o.pbase + u : -1;
     }
     count = 1;
     return o.pbase + o.pp + (p - o.pt);
@@ -247,12 +237,10 @@ __device__ __forceinline__ int32_t pack_of(const BucketOf &o, int32_t task, int3
 // ---------------------------------------------------------------- mode, order, packs
 // weight is read through the given pointer (global, or the fused kernel's LDS copy);
 // total = record count.  Leaves the selected mode in sh.mode.
-__device__ void stage_order_and_packs(const int32_t *weight, int32_t total, int32_t *order,
-                                      int32_t *pack_first, int32_t *pack_count, int32_t *num_packs,
-                                      int32_t *mode_out, const int32_t *rules, int32_t rule_count,
-                                      int32_t force, int32_t hkv, int32_t workers, int32_t buckets,
-                                      int32_t record_capacity, PlanShared &sh,
-                                      int16_t *order_mirror = nullptr) {
+__device__ void stage_order(const int32_t *weight, int32_t total, int32_t *order, int32_t *num_packs,
+                            int32_t *mode_out, const int32_t *rules, int32_t rule_count, int32_t force, int32_t hkv,
+                            int32_t workers, int32_t buckets, int32_t record_capacity, PlanShared &sh,
+                            int16_t *order_mirror = nullptr) {
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int per = (record_capacity + kPlanThreads - 1) / kPlanThreads;
     const int i0 = tid * per;
@@ -377,12 +365,18 @@ __device__ void stage_order_and_packs(const int32_t *weight, int32_t total, int3
         }
         lds_barrier();
     }
-    // Pack tables, one task per thread (consecutive threads, consecutive tasks: the
-    // stores of a wave land on neighbouring pack entries, not one record's Hkv tasks
-    // per lane): a task that starts a pack writes it.
+}
+
+// Pack tables, one task per thread (consecutive threads, consecutive tasks: the stores of a
+// wave land on neighbouring pack entries, not one record's Hkv tasks per lane): a task that
+// starts a pack writes it.  The single-stage kernel's; the fused one writes them with the
+// dispatch table (stage_units).
+__device__ void stage_packs(const int32_t *weight, const int32_t *order, int32_t total, int32_t *pack_first,
+                            int32_t *pack_count, int32_t hkv, int32_t buckets, const PlanShared &sh) {
     const int32_t ntasks = wmul(total, hkv);
-    for (int32_t task = tid; task < ntasks; task += kPlanThreads) {
-        const BucketOf o = bucket_at(sh, task / hkv, buckets);
+    for (int32_t task = threadIdx.x; task < ntasks; task += kPlanThreads) {
+        const int32_t j = (int32_t)((uint32_t)task / (uint32_t)hkv);
+        const BucketOf o = bucket_tables(sh, bucket_of(weight[order[j]], buckets));
         int32_t count;
         const int32_t unit = pack_of(o, task, hkv, count);
         if (unit >= 0) {
@@ -521,38 +515,59 @@ __device__ void stage_greedy_lists(const int32_t *weight, int32_t total, int32_t
     }
 }
 
-// ---------------------------------------------------------------- dispatch table
-// One entry per dispatch unit with its record resolved, so an attention launch goes
+// ---------------------------------------------------------------- units: packs and dispatch table
+// One dispatch entry per unit with its record resolved, so an attention launch goes
 // from a unit straight to its rows: {first task, tasks in the unit, request, split,
 // begin, end, kv group, kind}.  Units follow the mode the plan chose: tasks for R1
 // and STATIC (kind 1, task t is record t / Hkv: STATIC reads records directly and
-// R1's order is the identity, kernels/attention.py:41-47), packs for D1/D4 (kind 2,
-// pack u located in the bucket tables exactly as stage_order_and_packs lays the packs
-// out, its first record through the order).  Nothing is written for R0.  Everything
-// comes from LDS: record rec is (request_of(rec), rec - offsets[r]), with begin and end
-// computed as stage_emit_records computes them.
-__device__ void stage_dispatch_table(int32_t *table, int32_t capacity, const int16_t *order_mirror,
-                                     const RowMirror &rows, int32_t bcap, int32_t total, int32_t hkv,
-                                     int32_t buckets, const PlanShared &sh) {
+// R1's order is the identity, kernels/attention.py:41-47), packs for D1/D4 (kind 2),
+// located once for the pack tables and the entry.  Nothing is written for R0.
+//
+// Latency-bound, like the whole plan (one workgroup): per task, everything comes from LDS in
+// three reads -- the order, the record (`recs`, filled by the emission when the records fit
+// kLdsRecords; a search of the offsets otherwise), the bucket of its weight -- where a walk
+// over 16 bucket tables, twice, and a binary search stood before: 18.8 -> 11.8 us a build for 4100
+// tasks, 13.7 -> 9.7 for 1776 (launch included).
+constexpr int kLdsRecords = 2048;
+
+__device__ void stage_units(int32_t *table, int32_t capacity, int32_t *pack_first, int32_t *pack_count,
+                            const int16_t *order_mirror, const int4 *recs, const RowMirror &rows, int32_t bcap,
+                            int32_t total, const int32_t *weight, int32_t hkv, int32_t buckets, const PlanShared &sh) {
     const int32_t mode = sh.mode;
-    if (mode == 0) return;
-    // one task per thread, so a wave writes neighbouring entries (the Hkv lanes of a
-    // record find its request together: their LDS reads are broadcasts)
+    if (mode == 0 || (!table && mode == 1)) return;
+    // one task per thread, so a wave writes neighbouring entries (the Hkv lanes of a record
+    // read the same LDS words: broadcasts)
     const int32_t ntasks = wmul(total, hkv);
     for (int32_t task = threadIdx.x; task < ntasks; task += kPlanThreads) {
-        const int32_t j = task / hkv, g = task - j * hkv;
-        const int32_t rec = mode >= 3 ? (int32_t)order_mirror[j] : j;
-        const int32_t r = request_of(rows.offsets, bcap, rec);
-        const int32_t s = wadd(rec, -rows.offsets[r]);
-        const int32_t c = rows.chunk[r];
-        const int32_t b = wmul(s, c);
-        const int32_t e = min(wadd(b, c), rows.lengths[r]);
-        int32_t count = 1, unit = task;
-        if (mode >= 3) unit = pack_of(bucket_at(sh, j, buckets), task, hkv, count);
-        if (unit < 0 || unit >= capacity) continue;
+        const int32_t j = (int32_t)((uint32_t)task / (uint32_t)hkv), g = task - j * hkv;
+        int32_t rec = j, count = 1, unit = task;
+        if (mode >= 2) {  // (STATIC has pack tables too, and its units are tasks)
+            const int32_t sorted = order_mirror[j];
+            int32_t width;
+            const int32_t pack = pack_of(bucket_tables(sh, bucket_of(weight[sorted], buckets)), task, hkv, width);
+            if (pack >= 0) {
+                pack_first[pack] = task;
+                pack_count[pack] = width;
+            }
+            if (mode >= 3) {
+                rec = sorted;
+                unit = pack;
+                count = width;
+            }
+        }
+        if (!table || unit < 0 || unit >= capacity) continue;
+        int4 f;
+        if (recs) {
+            f = recs[rec];
+        } else {
+            const int32_t r = request_of(rows.offsets, bcap, rec);
+            const int32_t s = wadd(rec, -rows.offsets[r]);
+            const int32_t b = wmul(s, rows.chunk[r]);
+            f = make_int4(r, s, b, min(wadd(b, rows.chunk[r]), rows.lengths[r]));
+        }
         int32_t *ent = table + 8 * (int64_t)unit;
-        *reinterpret_cast<int4 *>(ent) = make_int4(task, count, r, s);
-        *reinterpret_cast<int4 *>(ent + 4) = make_int4(b, e, g, mode >= 3 ? 2 : 1);
+        *reinterpret_cast<int4 *>(ent) = make_int4(task, count, f.x, f.y);
+        *reinterpret_cast<int4 *>(ent + 4) = make_int4(f.z, f.w, g, mode >= 3 ? 2 : 1);
     }
 }
 
@@ -581,8 +596,11 @@ __global__ __launch_bounds__(kPlanThreads) void k_order_and_packs(
     int32_t *pack_count, int32_t *num_packs, int32_t *mode, const int32_t *rules, int32_t rule_count,
     int32_t force, int32_t hkv, int32_t workers, int32_t buckets, int32_t record_capacity) {
     __shared__ PlanShared sh;
-    stage_order_and_packs(weight, *record_count, order, pack_first, pack_count, num_packs, mode, rules,
-                          rule_count, force, hkv, workers, buckets, record_capacity, sh);
+    const int32_t total = *record_count;
+    stage_order(weight, total, order, num_packs, mode, rules, rule_count, force, hkv, workers, buckets, record_capacity,
+                sh);
+    __syncthreads();  // the order, in global memory
+    if (sh.mode >= 2) stage_packs(weight, order, total, pack_first, pack_count, hkv, buckets, sh);
 }
 
 __global__ __launch_bounds__(kPlanThreads) void k_greedy_lists(const int32_t *weight, const int32_t *record_count,
@@ -612,6 +630,10 @@ struct FusedLds {
     union {
         int32_t weight[kGreedyMaxRecords];
         uint32_t keys[kGreedyMaxRecords];
+        struct {
+            int32_t weight[kLdsRecords];
+            int4 recs[kLdsRecords];  // {request, split, begin, end}, with at most kLdsRecords records
+        } few;
     } b;
 };
 static_assert(sizeof(FusedLds) <= 160 * 1024, "fused plan LDS");
@@ -643,18 +665,15 @@ __global__ __launch_bounds__(kPlanThreads) void k_build_plan(sgd_plan_buffers p,
     }
     lds_barrier();
     const int32_t total = sh.record_count;
+    int4 *recs = total <= kLdsRecords ? L.b.few.recs : nullptr;
     stage_emit_by_record(mirror, total, p.batch_capacity, p.request, p.split, p.begin, p.end, p.weight, p.block_kv,
-                         L.b.weight);
+                         L.b.weight, recs);
     lds_barrier();
-    stage_order_and_packs(L.b.weight, total, p.order, p.pack_first, p.pack_count, p.num_packs, p.mode,
-                          rules_lds ? sh.rules : p.rules,
-                          p.rule_count, force, p.kv_heads, p.workers, p.buckets, p.batch_capacity * p.max_splits,
-                          sh, L.a.pre.order);
-    if (p.dispatch) {
-        lds_barrier();
-        stage_dispatch_table(p.dispatch, p.batch_capacity * p.max_splits * p.kv_heads, L.a.pre.order, mirror,
-                             p.batch_capacity, total, p.kv_heads, p.buckets, sh);
-    }
+    stage_order(L.b.weight, total, p.order, p.num_packs, p.mode, rules_lds ? sh.rules : p.rules, p.rule_count, force,
+                p.kv_heads, p.workers, p.buckets, p.batch_capacity * p.max_splits, sh, L.a.pre.order);
+    lds_barrier();
+    stage_units(p.dispatch, p.batch_capacity * p.max_splits * p.kv_heads, p.pack_first, p.pack_count, L.a.pre.order,
+                recs, mirror, p.batch_capacity, total, L.b.weight, p.kv_heads, p.buckets, sh);
     if (run_greedy) {
         lds_barrier();
         // the LPT's worker keys and tails take region A (free by now), its keys replace the weights
