@@ -3,7 +3,7 @@
 // token_to_kv_pool.set_kv_buffer does, integrations/sglang_backend.py:91-92) and the
 // step's q rows into the engine's stable per-layer query buffer (the qbuf.copy_ of
 // :102-103).  Upstream these are three device operations per layer (two scatters and
-// a copy); here one workgroup per token moves its 2 x Hkv x D + Hq x D 16-bit values
+// a copy); here one launch moves each token's 2 x Hkv x D + Hq x D 16-bit values
 // as 16-byte vector copies.
 //
 // The data is copied bit for bit (no dtype conversion); K/V rows go to the pool with
@@ -30,35 +30,32 @@ struct StoreArgs {
     int32_t loc64;
 };
 
-__device__ __forceinline__ void copy16(char *dst, const char *src) {
-    *reinterpret_cast<uint4 *>(dst) = *reinterpret_cast<const uint4 *>(src);
-}
-
+// Latency-bound (12 KB per token at the 8B shape): one 16-byte piece per thread, so that a
+// token's pieces are one round trip, made together with its slot's; with one workgroup per
+// token looping over them it was a round trip for the slot and one per 256 pieces: 1.3 us a
+// layer less in a 16-layer step of two tokens (64 / 8 heads), 0.6 at 48 tokens (32 / 8 heads).
 __global__ __launch_bounds__(kStoreThreads) void k_store_kv_stage_q(StoreArgs a) {
     const int32_t b = blockIdx.x;
     const int32_t kv_pieces = a.k_new ? a.hkv * a.chunks : 0;
     const int32_t q_pieces = a.q_in ? a.hq * a.chunks : 0;
-    int64_t slot = -1;
-    if (kv_pieces) {
-        slot = a.loc64 ? static_cast<const int64_t *>(a.loc)[b] : static_cast<const int32_t *>(a.loc)[b];
-        if (slot < 0 || slot >= a.cache_tokens) slot = -1;
-    }
     // pieces [0, kv) are K rows, [kv, 2 kv) V rows, then q rows; piece = (head, chunk)
-    for (int32_t p = threadIdx.x; p < 2 * kv_pieces + q_pieces; p += kStoreThreads) {
-        if (p < 2 * kv_pieces) {
-            if (slot < 0) continue;
-            const bool is_v = p >= kv_pieces;
-            const int32_t r = is_v ? p - kv_pieces : p;
-            const int32_t h = r / a.chunks, c = r - h * a.chunks;
-            const int64_t *ns = is_v ? a.vn : a.kn, *cs = is_v ? a.vc : a.kc;
-            const char *src = (is_v ? a.v_new : a.k_new) + b * ns[0] + h * ns[1] + c * 16;
-            char *dst = (is_v ? a.v_cache : a.k_cache) + slot * cs[0] + h * cs[1] + c * 16;
-            copy16(dst, src);
-        } else {
-            const int32_t r = p - 2 * kv_pieces;
-            const int32_t h = r / a.chunks, c = r - h * a.chunks;
-            copy16(a.q_out + b * a.qo[0] + h * a.qo[1] + c * 16, a.q_in + b * a.qi[0] + h * a.qi[1] + c * 16);
+    const int64_t pieces = 2 * (int64_t)kv_pieces + q_pieces;
+    for (int64_t p = (int64_t)blockIdx.y * kStoreThreads + threadIdx.x; p < pieces;
+         p += (int64_t)gridDim.y * kStoreThreads) {  // once, unless the grid's limit cut it
+        const bool is_q = p >= 2 * (int64_t)kv_pieces, is_v = !is_q && p >= kv_pieces;
+        const int32_t r = (int32_t)(is_q ? p - 2 * (int64_t)kv_pieces : is_v ? p - kv_pieces : p);
+        const int32_t h = (int32_t)((uint32_t)r / (uint32_t)a.chunks), c = r - h * a.chunks;
+        const int64_t *from = is_q ? a.qi : is_v ? a.vn : a.kn, *to = is_q ? a.qo : is_v ? a.vc : a.kc;
+        const char *src = (is_q ? a.q_in : is_v ? a.v_new : a.k_new) + b * from[0] + h * from[1] + c * 16;
+        char *dst = (is_q ? a.q_out : is_v ? a.v_cache : a.k_cache) + h * to[1] + c * 16;
+        const uint4 w = *reinterpret_cast<const uint4 *>(src);
+        int64_t row = b;
+        if (kv_pieces) {
+            const int64_t slot =
+                a.loc64 ? static_cast<const int64_t *>(a.loc)[b] : static_cast<const int32_t *>(a.loc)[b];
+            if (!is_q) row = slot >= 0 && slot < a.cache_tokens ? slot : -1;
         }
+        if (row >= 0) *reinterpret_cast<uint4 *>(dst + row * to[0]) = w;
     }
 }
 
@@ -118,6 +115,9 @@ extern "C" int sgd_store_kv_stage_q(const void *k_new, const void *v_new, const 
     }
     if (batch == 0 || (!kv && !q)) return 0;
     clear_stale_error();
-    hipLaunchKernelGGL(k_store_kv_stage_q, dim3(batch), dim3(kStoreThreads), 0, (hipStream_t)stream, a);
+    const int64_t pieces = (int64_t)a.chunks * ((kv ? 2 * (int64_t)kv_heads : 0) + (q ? query_heads : 0));
+    const int64_t parts = (pieces + kStoreThreads - 1) / kStoreThreads;
+    hipLaunchKernelGGL(k_store_kv_stage_q, dim3(batch, (unsigned)(parts < 65535 ? parts : 65535)), dim3(kStoreThreads), 0,
+                       (hipStream_t)stream, a);
     return launch_status("store_kv_stage_q");
 }
