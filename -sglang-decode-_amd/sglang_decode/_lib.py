@@ -106,12 +106,18 @@ def check(rc, what):
 
 
 def ptr(t):
-    """Device pointer of a tensor (None -> NULL)."""
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """Device pointer of a tensor (None -> NULL), as the entries' c_void_p arguments take it."""
+    return None if t is None else t.data_ptr()
+
+
+# The current stream's handle without a torch.cuda.Stream object around it.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def stream_handle(device=None):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    if _raw_stream is not None and device is not None and device.type == "cuda" and device.index is not None:
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def dtype_code(dtype):
