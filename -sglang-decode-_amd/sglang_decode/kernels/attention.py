@@ -54,12 +54,24 @@ def checked_layout(config, q, k, v, pages, indptr, out_dtype=None, who="execute"
             (0, 0), True)
 
 
+def plan_args(plan):
+    """A sgd_decode_args with the plan's pointers and configuration; the launch's own (q, K/V,
+    indices, strides, the layer's buffers) are left zero."""
+    a, c = _lib.DecodeArgsC(), plan.config
+    for name in ("lengths", "request", "split", "begin", "end", "order", "offsets", "chunk", "active",
+                 "record_count", "mode", "pack_first", "pack_count", "num_packs", "static_head", "static_next"):
+        setattr(a, name, getattr(plan, name).data_ptr())
+    a.query_heads, a.kv_heads, a.head_dim = c.query_heads, c.kv_heads, c.head_dim
+    a.max_splits, a.page_size, a.workers = c.max_splits, c.page_size, c.workers
+    return a
+
+
 def persistent_decode(plan, layer, q, k, v, pages, indptr, scale, k_strides, v_strides,
                       pt_strides, csr, kernel="auto", write_single=False):
     """One attention launch.  ``write_single``: the tasks that are their request's only
     split also write their row of ``layer.output`` (contiguous [Bcap, Hq, D] in q's dtype),
     so the merge may skip those rows (kernels.merge.merge_splits with min_splits 2)."""
-    a = plan.decode_args()
+    a = plan.decode_args() if hasattr(plan, "decode_args") else plan_args(plan)
     a.q, a.k, a.v = q.data_ptr(), k.data_ptr(), v.data_ptr()
     a.pages = pages.data_ptr()
     if indptr is not None:

@@ -1,0 +1,31 @@
+"""The C views a plan keeps (plan build and attention launch) follow a buffer or configuration
+that is put in another's place, and the attention's arguments take any object with a plan's fields."""
+import types
+
+import pytest
+
+from sglang_decode.config import DecodeConfig
+from sglang_decode.kernels.attention import plan_args
+from sglang_decode.runtime.workspace import PlanBuffers
+
+
+@pytest.mark.parametrize("field", ["lengths", "mode", "order", "static_head"])
+def test_views_follow_replaced_buffers(field):
+    c = DecodeConfig(batch_capacity=4, max_splits=2, max_context=256)
+    plan = PlanBuffers(c, "cpu")
+    plan.c_struct(), plan.decode_args()
+    other = getattr(plan, field).clone()
+    setattr(plan, field, other)
+    assert getattr(plan.c_struct(), field) == other.data_ptr()
+    assert getattr(plan.decode_args(), field) == other.data_ptr()
+    plan.config = DecodeConfig(batch_capacity=4, max_splits=2, max_context=256, workers=7)
+    assert plan.decode_args().workers == 7
+    lookalike = types.SimpleNamespace(**{k: v for k, v in vars(plan).items() if not k.startswith("_")})
+    assert bytes(plan_args(lookalike)) == bytes(plan.decode_args())
+
+
+def test_each_launch_has_its_own_arguments():
+    plan = PlanBuffers(DecodeConfig(batch_capacity=4, max_splits=2, max_context=256), "cpu")
+    a = plan.decode_args()
+    a.q, a.workers = 64, 1
+    assert plan.decode_args().q is None and plan.decode_args().workers == plan.config.workers
