@@ -1,6 +1,6 @@
 // Generic persistent paged GQA decode attention: any element strides (including
 // a non-unit head_dim stride), any 16-bit dtype, head_dim 64/128/256, group 1..16,
-// paged or CSR.  It is the fallback for layouts the tuned kernels do not take and
+// paged or CSR.  It is the fallback for layouts the pipelined kernel does not take and
 // the cross-check for them.
 //
 // Per task (record, kv head), kernels/attention.py:48-84: the group's q rows are

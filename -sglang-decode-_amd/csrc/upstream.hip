@@ -1,8 +1,8 @@
 // Upstream SGLang's two-stage split-KV decode, rebuilt for gfx950 as the comparator of
 // the reference's benchmark (benchmarks/baselines.py:8-34, which runs the pinned Triton
 // file third_party/sglang/decode_attention.py:245-601 of SGLang v0.4.6.post5).  It is the
-// schedule the persistent path replaces, so it uses the same VALU tile math
-// (valu_ops.h) and only the scheduling differs:
+// schedule the persistent path replaces, on the packed-dot-product tile math of valu_ops.h (the
+// persistent kernel's math runs on the matrix cores):
 //
 // stage 1: a grid of one workgroup per (split s < max_kv_splits, kv head, request b).
 //          Request b's L tokens are cut into chunks of c = ceil(ceil(L / S) / 32) * 32

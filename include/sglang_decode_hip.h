@@ -180,7 +180,8 @@ typedef struct sgd_decode_args {
     int32_t *counter;               /* per-layer claim counter, zero before the launch */
     int32_t *done_counter;          /* optional (may be NULL): workers that finished; the last
                                        one resets *counter and *done_counter to 0, so the pair is
-                                       zero again for the next launch */
+                                       zero again for the next launch.  Neither word is touched in
+                                       the modes that do not claim (R0, R1, STATIC) */
     const int32_t *static_head, *static_next;
     float *partial;                 /* [bcap, Hq, smax, D] */
     float *lse;                     /* [bcap, Hq, smax] */
