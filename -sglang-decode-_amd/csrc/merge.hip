@@ -94,8 +94,11 @@ __global__ __launch_bounds__(64 * kSplitWaves) void k_merge(const float *__restr
 
 // The rows of requests with no split or at least min_splits of them (all rows on a plan
 // error): at most one residency round of workgroups (the occupancy API's count per CU),
-// striding over the rows in (request, head) order.  A row of 1 <= n < min_splits splits (written by the attention) costs its
-// workgroup only the split count, which is requested a row ahead.
+// striding over the rows in (request, head) order.  A row of 1 <= n < min_splits splits
+// (written by the attention) is nothing but its count to read, so the counts of a workgroup's
+// next 64 rows come in one load, a lane each, and only the rows to merge are walked: those that
+// a wave merges alone, dealt to the waves, then the long ones.  Row after row, each waiting
+// for its count, 20992 rows (128 heads of D 256, 123 of 164 requests) took 23.0 us; now 9.7.
 template <int DT, int DPL>
 __global__ __launch_bounds__(64 * kSplitWaves) void k_merge_rows(const float *__restrict__ partial,
                                                                  const float *__restrict__ lse,
@@ -106,17 +109,24 @@ __global__ __launch_bounds__(64 * kSplitWaves) void k_merge_rows(const float *__
     __shared__ float sm[kSplitWaves], sd[kSplitWaves], sacc[kSplitWaves][DPL * 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const bool bad = *error != 0;
-    int32_t row = blockIdx.x;
-    int32_t n = row < rows ? __builtin_amdgcn_readfirstlane(counts[row / hq]) : 0;
-    while (row < rows) {  // uniform over the workgroup
-        const int32_t next = row + gridDim.x;
-        const int32_t n_next = next < rows ? __builtin_amdgcn_readfirstlane(counts[next / hq]) : 0;
-        if (bad || n == 0 || n >= min_splits) {
-            merge_one<DT, DPL>(partial, lse, n, bad, out, row, smax, sm, sd, sacc, lane, wave);
-            if (next < rows) lds_barrier();  // the LDS combine of this row is read before the next one's
+    for (int64_t base = blockIdx.x; base < rows; base += 64 * (int64_t)gridDim.x) {  // uniform over the workgroup
+        const int64_t mine = base + lane * (int64_t)gridDim.x;
+        const int32_t n_mine = mine < rows ? counts[(uint32_t)mine / (uint32_t)hq] : 1;
+        const bool todo = mine < rows && (bad || n_mine == 0 || n_mine >= min_splits);
+        uint64_t alone = __ballot(todo && n_mine <= kRowsInFlight);
+        uint64_t split = __ballot(todo && n_mine > kRowsInFlight);
+        for (int k = 0; alone; ++k, alone &= alone - 1) {
+            if (k % kSplitWaves != wave) continue;
+            const int at = __builtin_ctzll(alone);
+            merge_row<DT, DPL>(partial, lse, __builtin_amdgcn_readlane(n_mine, at), bad, out,
+                               base + at * (int64_t)gridDim.x, smax, lane);
         }
-        row = next;
-        n = n_next;
+        for (; split; split &= split - 1) {
+            const int at = __builtin_ctzll(split);
+            merge_one<DT, DPL>(partial, lse, __builtin_amdgcn_readlane(n_mine, at), bad, out,
+                               base + at * (int64_t)gridDim.x, smax, sm, sd, sacc, lane, wave);
+            lds_barrier();  // the LDS combine of this row is read before the next one's
+        }
     }
 }
 
