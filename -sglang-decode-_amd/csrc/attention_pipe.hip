@@ -38,12 +38,25 @@
 //                    tiles that raise some head's maximum.  (Letting scores exceed the maximum
 //                    by 2^8 first is no faster, and the largest p is then not the 1 that rounds
 //                    exactly: 2.2e-3 instead of 1.75e-3 off in bf16, 1.66e-3 of it the result's own
-//                    rounding.)  P is rounded to the KV dtype (kernels/attention.py:78).
+//                    rounding.)  P is rounded to the KV dtype (kernels/attention.py:78), and where
+//                    fewer waves share a task than would keep that error down its remainder
+//                    is multiplied too (below).
 //   O^T += V^T . P^T the B operand is P as S^T left it; the A operand needs one dim of each of
 //                    the lane group's tokens per lane: lane (m, j) loads kRowDims consecutive dims
 //                    of each of its tokens and block b takes element b (v_perm), so output row r
 //                    of block b is dim kRowDims r + b (D = 256: 128 h + 8 r + b).
 // The next tile's rows are requested into the registers this tile's free up, V after P.V.
+//
+// The remainder of P: a wave's largest p is 1 and rounds exactly, the other p of the heavy tokens do
+// not, so the fewer waves share a task the larger the error of the rounded P: against 64 bits, in bf16 before
+// the output's rounding, 4.6e-4 with eight waves (groups up to 4 in an earlier kernel), 5.8e-4 with
+// four, 6.2e-4 with three.  So groups up to 4, and head_dim 256 (three waves), multiply
+// P - round(P) in the KV dtype as well, which leaves 1e-6.  Groups up to 4 leave the MFMA's upper 8
+// columns free: column n + 8 takes the remainders of head n, at no MFMA more, and they go to merge rows of
+// their own (added in registers at the task's end: 0.6 to 1.1 us a launch more).  8 and 16 heads at D = 256, which
+// have no LDS for such rows, take a second MFMA a block into accumulators of their own.  It costs up to 2 %
+// of a layer's time for groups up to 4 (eight layers of 64 requests 640 -> 642 us, a layer of 128 of ~60 tokens 24.9 -> 25.6),
+// 1 to 7 % for the others (48 requests of ~1000 tokens, D 256: 8 heads 86.1 -> 87.0, 16 heads 60.9 -> 63.7).
 //
 // Geometry: two workgroups must be resident per CU (the default worker count), and the hardware
 // deals a workgroup's waves to the SIMDs in turn, so five waves take two slots of one SIMD:
@@ -51,6 +64,8 @@
 // at D = 256, where a tile and its output are 128 registers, 3 + 1 waves have 256.  At 16 tokens a
 // tile D = 128 fits 8 + 1 waves only with spills: 75 us for the first layer above.  64-token
 // tiles at D = 64 (4 + 1 waves): 57.0 against 52.9 us.
+#include <float.h>
+
 #include "valu_ops.h"
 
 namespace sgd {
@@ -111,7 +126,7 @@ struct PipeShared {
     int32_t idx[2][PGeo<D>::kTile * PGeo<D>::kWaves];  // page/slot indices of the first kWaves tiles
     float m[2][PGeo<D>::kWaves][16], d[2][PGeo<D>::kWaves][16];
     int32_t indptr[kIndptrLds];
-    // then q rows [2][G][kQRow bytes] and merge rows [merge_sets(G)][kWaves][pass_heads(G)][kORow]
+    // then q rows [2][G][kQRow bytes] and merge rows [merge_sets(G)][kWaves][merge_heads(G)][kORow]
 };
 
 // The merge rows share a CU's 160 KB with a second workgroup: two sets, alternating by task
@@ -127,10 +142,21 @@ __host__ __device__ constexpr int merge_sets(int g) { return g <= (D == 256 ? 4 
 template <int D>
 __host__ __device__ constexpr int merge_barriers(int g) { return merge_sets<D>(g) == 2 ? 1 : 2 * (g / pass_heads<D>(g)); }
 
+// How a task's remainders of P are multiplied (above).
+enum Rest { kNoRest, kRestColumns, kRestOwn };
+template <int D>
+__host__ __device__ constexpr Rest rest_form(int g) { return g <= 4 ? kRestColumns : D == 256 ? kRestOwn : kNoRest; }
+
+// Rows of a wave's share of the merge: those of the remainders after the heads'.
+template <int D>
+__host__ __device__ constexpr int merge_heads(int g) {
+    return rest_form<D>(g) == kRestColumns ? 2 * g : pass_heads<D>(g);
+}
+
 template <int D>
 __host__ __device__ constexpr int pipe_lds_bytes(int g) {
     return (int)sizeof(PipeShared<D>) + 2 * g * PGeo<D>::kQRow +
-           merge_sets<D>(g) * PGeo<D>::kWaves * pass_heads<D>(g) * PGeo<D>::kORow * (int)sizeof(float);
+           merge_sets<D>(g) * PGeo<D>::kWaves * merge_heads<D>(g) * PGeo<D>::kORow * (int)sizeof(float);
 }
 template <int D>
 constexpr bool two_per_cu() {
@@ -345,19 +371,31 @@ __device__ __forceinline__ void issue_v(const sgd_decode_args &a, const Source &
 }
 
 // A wave's softmax state and output: lane (n, j) holds head n's maximum and its own tokens'
-// share of the denominator, and dims of rows 4j + i of each O^T block.
-template <int D>
+// share of the denominator, and dims of rows 4j + i of each O^T block (kRestOwn: of the remainders too).
+template <int D, Rest kRest>
 struct State {
     float m, den;
     f32x4 o[PGeo<D>::kBlocks];
+    f32x4 rest[kRest == kRestOwn ? PGeo<D>::kBlocks : 1];
 };
+
+// a - its value in the KV dtype, for both halves of a packed pair; where `keep` is 0 the pair itself.
+template <int DT>
+__device__ __forceinline__ uint32_t remainder2(uint32_t w, float lo, float hi, uint32_t keep) {
+    w &= keep;
+    return valu::pack2<DT>(lo - to_f32<DT>(w & 0xffff), hi - to_f32<DT>(w >> 16));
+}
+
+// The remainders' share of an output, to add to that of the rounded P.  An infinite V row makes the latter
+// infinite, which 0 x infinity or an infinity of the other sign here must not turn into NaN.
+__device__ __forceinline__ float finite(float rest) { return __builtin_amdgcn_fmed3f(rest, -FLT_MAX, FLT_MAX); }
 
 // One tile of nvalid tokens, whose rows are in (or on their way to) r; the tile at `s` is
 // requested into the same registers as they become free.
-template <int DT, bool CSR, int D, bool kPow2>
+template <int DT, bool CSR, int D, bool kPow2, Rest kRest>
 __device__ __forceinline__ void tile_step(const sgd_decode_args &a, TileRegs<D> &r, char *stage, const char *q,
                                           int32_t nvalid, float scale2, const Source &s, const PageMap<kPow2> &pm,
-                                          int lane, State<D> &st) {
+                                          int lane, State<D, kRest> &st) {
     using G = PGeo<D>;
     constexpr int kV = G::kVals;
     // per-lane positions are rebuilt each tile, not held live
@@ -406,7 +444,10 @@ __device__ __forceinline__ void tile_step(const sgd_decode_args &a, TileRegs<D> 
         st.m = m_new;
         st.den *= alpha;
 #pragma unroll
-        for (int b = 0; b < G::kBlocks; ++b) st.o[b] = st.o[b] * alpha;
+        for (int b = 0; b < G::kBlocks; ++b) {
+            st.o[b] = st.o[b] * alpha;
+            if constexpr (kRest == kRestOwn) st.rest[b] = st.rest[b] * alpha;
+        }
     }
     float p[kV];
 #pragma unroll
@@ -417,6 +458,15 @@ __device__ __forceinline__ void tile_step(const sgd_decode_args &a, TileRegs<D> 
     uint32_t pw[kV / 2];  // P in the KV dtype, token pairs
 #pragma unroll
     for (int i = 0; i < kV; i += 2) pw[i / 2] = valu::pack2<DT>(p[i], p[i + 1]);
+    uint32_t rest[kRest == kRestOwn ? kV / 2 : 1];
+    if constexpr (kRest == kRestOwn) {
+#pragma unroll
+        for (int i = 0; i < kV; i += 2) rest[i / 2] = remainder2<DT>(pw[i / 2], p[i], p[i + 1], 0xffffffffu);
+    } else if constexpr (kRest == kRestColumns) {
+        const uint32_t keep = m & 8 ? 0xffffffffu : 0u;
+#pragma unroll
+        for (int i = 0; i < kV; i += 2) pw[i / 2] = remainder2<DT>(pw[i / 2], p[i], p[i + 1], keep);
+    }
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (!G::kEarlyK) issue_k<CSR, D>(a, s, pm, lane, r);
     __builtin_amdgcn_sched_barrier(0);
@@ -428,11 +478,15 @@ __device__ __forceinline__ void tile_step(const sgd_decode_args &a, TileRegs<D> 
         for (int b = 0; b < G::kBlocks; ++b) {
             const uint32_t sel = (b & 1) ? 0x07060302u : 0x05040100u;
             auto pair = [&](int i) { return __builtin_amdgcn_perm(r.v[t + i + 1][b >> 1], r.v[t + i][b >> 1], sel); };
-            if constexpr (kV >= 8)
+            if constexpr (kV >= 8) {
+                static_assert(kV < 8 || kRest != kRestOwn, "remainders in a second MFMA: the 16-token tile's");
                 st.o[b] = mfma32<DT>(make_uint4(pair(0), pair(2), pair(4), pair(6)),
                                      make_uint4(pk[0], pk[1], pk[2], pk[3]), st.o[b]);
-            else
-                st.o[b] = mfma16<DT>(make_uint2(pair(0), pair(2)), make_uint2(pk[0], pk[1]), st.o[b]);
+            } else {
+                const uint2 v = make_uint2(pair(0), pair(2));
+                st.o[b] = mfma16<DT>(v, make_uint2(pk[0], pk[1]), st.o[b]);
+                if constexpr (kRest == kRestOwn) st.rest[b] = mfma16<DT>(v, make_uint2(rest[0], rest[1]), st.rest[b]);
+            }
         }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -583,7 +637,7 @@ __device__ __forceinline__ void helper_wave(const sgd_decode_args &a, PipeShared
 }
 
 // ------------------------------------------------------------------ kernel
-template <int DT, bool CSR, int D, bool kOut, bool kPow2, bool kPasses>
+template <int DT, bool CSR, int D, bool kOut, bool kPow2, Rest kRest, bool kPasses>
 __global__ __launch_bounds__(PGeo<D>::kThreads, PGeo<D>::kWavesPerSimd) void k_attention_pipe(sgd_decode_args a) {
     using GG = PGeo<D>;
     constexpr int kTile = GG::kTile, kWaves = GG::kWaves;
@@ -600,7 +654,9 @@ __global__ __launch_bounds__(PGeo<D>::kThreads, PGeo<D>::kWavesPerSimd) void k_a
     }
     const float scale2 = a.scale * kLog2e;
     const int32_t heads = kPasses ? pass_heads<D>(G) : G;  // kPasses: G > heads per merge pass
-    const bool one_set = merge_sets<D>(G) == 1;
+    // kRestColumns: groups up to 4; kRestOwn: 8 and 16 heads at D = 256
+    const bool one_set = kRest == kNoRest ? merge_sets<D>(G) == 1 : kRest == kRestOwn;
+    const int32_t row_heads = kRest == kRestColumns ? 2 * heads : heads;  // merge_heads
 
     auto read_slot = [&](int32_t k) {
         const Slot s = sh.slot[k & 1];
@@ -620,7 +676,7 @@ __global__ __launch_bounds__(PGeo<D>::kThreads, PGeo<D>::kWavesPerSimd) void k_a
 #pragma unroll
         for (int h = 0; h < GG::kHalves; ++h) r.idx[h] = ix[16 * h + 4 * j + (m & 3)];
     };
-    auto merge_rows = [&](int par) { return so + (one_set ? 0 : par) * kWaves * heads * GG::kORow; };
+    auto merge_rows = [&](int par) { return so + (one_set ? 0 : par) * kWaves * row_heads * GG::kORow; };
     // The waves' states of task t's heads h0 .., merged in wave order.  A request's first split also writes
     // its normalized rows to `out` (kOut: sgd_decode_args.out set) -- final for a single-split
     // request, overwritten by the merge otherwise.
@@ -632,13 +688,16 @@ __global__ __launch_bounds__(PGeo<D>::kThreads, PGeo<D>::kWavesPerSimd) void k_a
             float mm = -INFINITY;
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) mm = fmaxf(mm, sh.m[par][w][h]);
-            float dd = 0.f, acc = 0.f;
+            float dd = 0.f, acc = 0.f, rest = 0.f;
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) {
                 const float f = __builtin_amdgcn_exp2f(sh.m[par][w][h] - mm);
+                const float *o = rows + (w * row_heads + h - h0) * GG::kORow + merge_pos<D>(d);
                 dd += sh.d[par][w][h] * f;
-                acc += rows[(w * heads + h - h0) * GG::kORow + merge_pos<D>(d)] * f;
+                acc += *o * f;
+                if constexpr (kRest == kRestColumns) rest += o[heads * GG::kORow] * f;
             }
+            if constexpr (kRest == kRestColumns) acc += finite(rest);
             const int64_t row = (int64_t)t.request * a.query_heads + t.group * G + h;
             const int64_t slot = row * a.max_splits + t.split;
             a.partial[slot * D + d] = acc / dd;
@@ -673,11 +732,14 @@ __global__ __launch_bounds__(PGeo<D>::kThreads, PGeo<D>::kWavesPerSimd) void k_a
         cur = nxt;
         const int32_t n0 = n1;
         const char *q = sq + (par * G + (lane & 15 & (G - 1))) * GG::kQRow + (lane >> 4) * 16;
-        State<D> st;
+        State<D, kRest> st;
         st.m = -INFINITY;
         st.den = 0.f;
 #pragma unroll
-        for (int b = 0; b < GG::kBlocks; ++b) st.o[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int b = 0; b < GG::kBlocks; ++b) {
+            st.o[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (kRest == kRestOwn) st.rest[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
         bool known = false;  // nxt holds task k + 1
         requested = false;
         int32_t tok = cur.start + wave * kTile;
@@ -704,13 +766,29 @@ __global__ __launch_bounds__(PGeo<D>::kThreads, PGeo<D>::kWavesPerSimd) void k_a
                     if (requested) first_tile(nxt, k + 1, lane);
                 }
             }
-            tile_step<DT, CSR, D, kPow2>(a, r, sh.kstage[wave], q, min(kTile, cur.end - tok), scale2, src, pm, lane,
-                                         st);
+            tile_step<DT, CSR, D, kPow2, kRest>(a, r, sh.kstage[wave], q, min(kTile, cur.end - tok), scale2, src, pm,
+                                                lane, st);
         }
 
         // ---- the wave's state to LDS, then the merge
         st.den += __shfl_xor(st.den, 16, 64);
         st.den += __shfl_xor(st.den, 32, 64);
+        if constexpr (kRest == kRestOwn) {
+            // Straight-line code that a launch's first task fetches: the clamps stay out of it.
+            float top = 0.f;
+#pragma unroll
+            for (int b = 0; b < GG::kBlocks; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) top = fmaxf(top, __builtin_fabsf(st.o[b][i]));
+            if (__builtin_expect(__ballot(top == INFINITY) != 0, 0)) {
+#pragma unroll
+                for (int b = 0; b < GG::kBlocks; ++b)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) st.rest[b][i] = finite(st.rest[b][i]);
+            }
+#pragma unroll
+            for (int b = 0; b < GG::kBlocks; ++b) st.o[b] = st.o[b] + st.rest[b];
+        }
         const int n = lane & 15, j = lane >> 4;
         if (j == 0) {
             sh.m[par][wave][n] = st.m;
@@ -718,8 +796,10 @@ __global__ __launch_bounds__(PGeo<D>::kThreads, PGeo<D>::kWavesPerSimd) void k_a
         }
         for (int32_t h0 = 0;; h0 += heads) {
             if (one_set) lds_barrier();  // the rows' last merge has read them
-            if (n >= h0 && n < h0 + heads) {
-                float *dst = merge_rows(par) + (wave * heads + n - h0) * GG::kORow;
+            // the lane's row: its column's head, or that head's remainders
+            const int row = kRest != kRestColumns ? n - h0 : n & 8 ? heads + (n & 7) : n;
+            if (kRest != kRestColumns ? n >= h0 && n < h0 + heads : (n & 7) < heads) {
+                float *dst = merge_rows(par) + (wave * row_heads + row) * GG::kORow;
 #pragma unroll
                 for (int b = 0; b < GG::kBlocks; ++b)
                     *reinterpret_cast<f32x4 *>(dst + 128 * (b / GG::kRowDims) + 4 * GG::kRowDims * j +
@@ -734,25 +814,28 @@ __global__ __launch_bounds__(PGeo<D>::kThreads, PGeo<D>::kWavesPerSimd) void k_a
     }
 }
 
-template <int DT, bool CSR, int D, bool kOut, bool kPow2, bool kPasses>
+template <int DT, bool CSR, int D, bool kOut, bool kPow2, Rest kRest, bool kPasses>
 int launch_pipe_o(const sgd_decode_args &a, hipStream_t stream) {
     static bool attr[kOnceDevices] = {};
     const int bytes = pipe_lds_bytes<D>(a.query_heads / a.kv_heads);
-    if (int rc = set_dynamic_lds((const void *)k_attention_pipe<DT, CSR, D, kOut, kPow2, kPasses>, 80 * 1024, attr,
+    if (int rc = set_dynamic_lds((const void *)k_attention_pipe<DT, CSR, D, kOut, kPow2, kRest, kPasses>, 80 * 1024, attr,
                                  "pipelined attention"))
         return rc;
-    hipLaunchKernelGGL((k_attention_pipe<DT, CSR, D, kOut, kPow2, kPasses>), dim3(a.workers), dim3(PGeo<D>::kThreads), bytes,
-                       stream, a);
+    hipLaunchKernelGGL((k_attention_pipe<DT, CSR, D, kOut, kPow2, kRest, kPasses>), dim3(a.workers),
+                       dim3(PGeo<D>::kThreads), bytes, stream, a);
     return launch_status("persistent_decode(pipelined)");
 }
 
 template <int DT, bool CSR, int D, bool kOut, bool kPow2>
 int launch_pipe_g(const sgd_decode_args &a, hipStream_t stream) {
-    if constexpr (D == 256) {
-        const int g = a.query_heads / a.kv_heads;
-        if (g > pass_heads<D>(g)) return launch_pipe_o<DT, CSR, D, kOut, kPow2, true>(a, stream);
-    }
-    return launch_pipe_o<DT, CSR, D, kOut, kPow2, false>(a, stream);
+    const int g = a.query_heads / a.kv_heads;
+    if (rest_form<D>(g) == kRestColumns)
+        return launch_pipe_o<DT, CSR, D, kOut, kPow2, kRestColumns, false>(a, stream);
+    if constexpr (D == 256)
+        return g > pass_heads<D>(g) ? launch_pipe_o<DT, CSR, D, kOut, kPow2, kRestOwn, true>(a, stream)
+                                    : launch_pipe_o<DT, CSR, D, kOut, kPow2, kRestOwn, false>(a, stream);
+    else
+        return launch_pipe_o<DT, CSR, D, kOut, kPow2, kNoRest, false>(a, stream);
 }
 
 // A power-of-two page (CSR's page of one token included) maps tokens by shift and mask;

@@ -305,6 +305,7 @@ inline void launch(const char *name, void (*k)(P...), dim3 grid, dim3 block, siz
 #define __builtin_amdgcn_fdot2(a, b, c, clamp) ::emu::dot2(1, (a), (b), (c))
 #define __builtin_amdgcn_perm(a, b, s) ::emu::perm((a), (b), (s))
 #define __builtin_amdgcn_exp2f(x) exp2f(x)
+#define __builtin_amdgcn_fmed3f(x, lo, hi) fminf(fmaxf((x), (lo)), (hi))
 #define __builtin_amdgcn_rcpf(x) (1.0f / (x))
 #define __builtin_amdgcn_kernarg_segment_ptr() (::emu::fatal("kernarg_segment_ptr is not emulated"), (void *)nullptr)
 #define __hip_atomic_fetch_add(p, v, o, s) ::emu::atomic_fetch_add((p), (v))

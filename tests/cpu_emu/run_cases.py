@@ -16,6 +16,9 @@ Two more case kinds drive the entry points outside the engine's path:
 oracle; {"noalloc": workload, "batches": [[n, shrink], ...], "mode": m} runs
 sgd_decode_noalloc on consecutive calls (the first n requests, contexts divided by
 shrink) and compares each bitwise with the allocating entry points on the same inputs.
+
+{"precision": [group, head_dim], "dtype": ...} gives the relative 2-norm error of the attention's
+fp32 split slots against 64 bits, before any rounding of an output.
 """
 import json
 import os
@@ -249,6 +252,29 @@ def _merge_min(emu, bcap, hq, smax, d, min_splits):
                 error_nan=bool(np.isnan(D.from_bits16(res["error"], _lib.SGD_BF16)).all()))
 
 
+def _precision(emu, group, d, dtype):
+    import numpy as np
+    import driver as D
+    from sglang_decode import workloads as W
+    from sglang_decode.config import DecodeConfig
+    lengths, splits = [300, 517, 1000], [1, 2, 3]
+    c = DecodeConfig(batch_capacity=3, max_splits=3, max_context=1024, query_heads=group, kv_heads=1, head_dim=d,
+                     page_size=1, workers=6)
+    q, k, v, indptr, indices = W.make_csr_inputs(c, lengths, seed=group + d, dtype=dtype, device="cpu")
+    q = q * 2  # scores of standard deviation 2
+    r = D.decode(emu, c, lengths, splits, q, k, v, indices, indptr, mode=1)
+    p, num, den = r["plan"], 0.0, 0.0
+    for i in range(p["record_count"]):
+        row, rows = p["request"][i], indices[int(indptr[p["request"][i]]):].long()[p["begin"][i]:p["end"][i]]
+        s = q[row].double().numpy() @ k[rows, 0].double().numpy().T * d ** -0.5
+        w = np.exp(s - s.max(1, keepdims=True))
+        exact = (w / w.sum(1, keepdims=True)) @ v[rows, 0].double().numpy()
+        num += ((r["partial"][row, :, p["split"][i]] - exact) ** 2).sum()
+        den += (exact ** 2).sum()
+    return dict(case="precision", group=group, head_dim=d, dtype=str(dtype), kernel=r["kernel"],
+                records=p["record_count"], error=float((num / den) ** 0.5))
+
+
 def run(cases, asan):
     import torch
     import driver as D
@@ -261,6 +287,8 @@ def run(cases, asan):
             lengths, smax = case["upstream"]
             print(json.dumps(_upstream(emu, list(lengths), int(smax), getattr(torch, case.get("dtype", "bfloat16")))),
                   flush=True)
+        elif "precision" in case:
+            print(json.dumps(_precision(emu, *case["precision"], getattr(torch, case["dtype"]))), flush=True)
         elif "merge_min" in case:
             bcap, hq, smax, d, m = case["merge_min"]
             print(json.dumps(_merge_min(emu, int(bcap), int(hq), int(smax), int(d), int(m))), flush=True)

@@ -145,6 +145,22 @@ def test_few_workers_walk_long_task_chains(asan_build):
     _assert_clean(rc, rows, err, 10 + 1 + 1)
 
 
+def test_probabilities_are_held_beyond_the_kv_dtype(asan_build):
+    """The fp32 split slots against 64 bits, for the groups and head dims that deal a task to fewer
+    waves than eight (groups up to 4) or four (head_dim 256).  A wave's largest probability is an exact 1, so with
+    probabilities of 16 bits alone the error grows as the waves get fewer (bf16: 4.7e-4 with eight,
+    6e-4 with four); held as a rounded value and its remainder they are off by 2^-18 at most (fp16: or
+    2^-25 of the largest), and the slots by that, fp32 rounding and the exponential's 1e-6."""
+    cases = [{"precision": [g, d], "dtype": t} for g, d, t in
+             ((1, 64, "float16"), (4, 64, "bfloat16"), (2, 128, "float16"), (4, 128, "bfloat16"), (1, 256, "bfloat16"),
+              (4, 256, "float16"), (8, 256, "bfloat16"), (16, 256, "bfloat16"), (16, 256, "float16"))]
+    rc, rows, err = _run(cases)
+    assert rc == 0 and "ERROR: AddressSanitizer" not in err, err[-4000:]
+    assert len(rows) == len(cases), err[-2000:]
+    for r in rows:
+        assert r["kernel"] != "generic" and r["records"] == 6 and r["error"] < 1e-5, r
+
+
 def test_upstream_comparator_and_no_alloc_entry_in_bounds(asan_build):
     """The two entry points outside the engine's path.  sgd_upstream_decode (the upstream
     two-stage split-KV comparator): empty, 1-token and 700-token rows over 16 splits, a

@@ -2,8 +2,8 @@
 the FP32 oracle (2e-2 abs / 1e-2 rel): scores spanning hundreds of log units (the online
 softmax must rescale its running state from tile to tile and split to split without
 overflow), one dominant token anywhere in a row (the output is that token's V row), all
-keys equal (the output is the mean of the V rows), and large V values in fp16 (fp32
-accumulation, one rounding at the end).  Every kernel that takes the shape runs each case,
+keys equal (the output is the mean of the V rows), large V values in fp16 (fp32
+accumulation, one rounding at the end), and infinite ones.  Every kernel that takes the shape runs each case,
 with several splits per request so the merge combines states of very different maxima."""
 import pytest
 import torch
@@ -111,3 +111,25 @@ def test_large_values_fp16():
         out = run(c, kernel, q, k, v, indptr, indices, LENGTHS, dtype)
         assert torch.isfinite(out[:len(LENGTHS)].float()).all(), kernel
         close(out[:len(LENGTHS)], expected[:len(LENGTHS)], atol=2e-2 * vscale, msg=kernel)
+
+
+@pytest.mark.parametrize("group,d", [(1, 64), (4, 128), (8, 128), (4, 256), (8, 256), (16, 256)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_infinite_v_stays_infinite(group, d, dtype):
+    """One infinite element in a V row that every head weighs: that output is the infinity, its
+    neighbours the mean of V.  Equal keys make every probability an exact 1, whose remainder in the KV
+    dtype is 0, and 0 x infinity must not reach the output."""
+    c = DecodeConfig(batch_capacity=2, max_splits=2, max_context=512, query_heads=2 * group, kv_heads=2, head_dim=d,
+                     page_size=1, workers=8)
+    lengths = [300, 33]
+    q, k, v, indptr, indices = W.make_csr_inputs(c, lengths, seed=9, dtype=dtype)
+    k.copy_(k[:1].expand_as(k))
+    slots = [indices[:300].long(), indices[300:333].long()]
+    v[slots[0][17], 0, 3] = float("inf")
+    v[slots[1][32], 1, d - 1] = float("-inf")
+    for kernel in kernels(group):
+        print(f"infinite V group={group} d={d} dtype={dtype} kernel={kernel}", flush=True)
+        out = run(c, kernel, q, k, v, indptr, indices, lengths, dtype)
+        for r in range(2):
+            expected = v[slots[r]].float().mean(0).repeat_interleave(group, 0).cpu().numpy()
+            close(out[r], expected, msg=f"{kernel} request {r}")
