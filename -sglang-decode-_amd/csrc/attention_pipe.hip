@@ -556,11 +556,16 @@ __device__ __forceinline__ void helper_wave(const sgd_decode_args &a, PipeShared
                                  : iptr_ready && info.request < iptr_n ? uni(sh.indptr[info.request])
                                                                        : uni(a.indptr[info.request]);
             const int32_t *rows = CSR ? a.pages + ind0 : a.pages + (int64_t)info.request * a.pt_stride[0];
+            // A record without a token has no last one to repeat (end - 1 may lie before the table), and
+            // nothing uses its indices: it reads a word that is there.  (A branch cost up to 47 SGPR spills.)
+            const bool some = info.end > info.start;
+            rows = some ? rows : a.mode;
+            const int32_t last = some ? info.end - 1 : 0;
             constexpr int kIdx = GG::kTile * GG::kWaves, kLoads = (kIdx + 63) / 64;
             int32_t tile_idx[kLoads];
 #pragma unroll
             for (int t = 0; t < kLoads; ++t) {
-                const int32_t tok = min(info.start + 64 * t + lane, info.end - 1);
+                const int32_t tok = min(info.start + 64 * t + lane, last);
                 tile_idx[t] = CSR ? rows[tok] : rows[(int64_t)pm.page(tok) * a.pt_stride[1]];
             }
             // the group's q rows, 16 B pieces (head = piece / (D / 8))

@@ -121,9 +121,10 @@ class Plan:
 
 
 def decode(emu, config, lengths, splits, q, k, v, pages, indptr=None, *, mode=-1, kernel="auto", scale=None,
-           rules=(), run_greedy=None, poison=True, direct=True):
+           rules=(), run_greedy=None, poison=True, direct=True, edit=None):
     """One prepare() + execute() on the executor.  q/k/v: torch CPU tensors (bf16/fp16);
     pages: paged table [Bcap, max_pages] or CSR kv_indices; indptr: CSR kv_indptr or None.
+    ``edit(plan)`` changes the built plan before the attention reads it.
     Returns dict(out [Bcap,Hq,D] float32, partial, lse, plan, kernel)."""
     import torch
     c = config
@@ -143,6 +144,8 @@ def decode(emu, config, lengths, splits, q, k, v, pages, indptr=None, *, mode=-1
         run_greedy = int(mode) == 2 or any(int(r.mode) == 2 for r in rules)
     emu.check(emu.lib.sgd_build_plan(ctypes.byref(plan.c_struct()), int(mode), int(bool(run_greedy)),
                                      ptr(sync), 2, None), "build_plan")
+    if edit is not None:
+        edit(plan)
     qd, kd, vd = emu.upload(bits16(q)), emu.upload(bits16(k)), emu.upload(bits16(v))
     pd = emu.upload(pages.detach().cpu().numpy().astype(np.int32))
     ipd = emu.upload(indptr.detach().cpu().numpy().astype(np.int32)) if indptr is not None else None

@@ -17,6 +17,10 @@ oracle; {"noalloc": workload, "batches": [[n, shrink], ...], "mode": m} runs
 sgd_decode_noalloc on consecutive calls (the first n requests, contexts divided by
 shrink) and compares each bitwise with the allocating entry points on the same inputs.
 
+{"spans": [[begin, end], ...], "page": p, "dispatch": b} gives the plan's first records (one a request)
+other spans than the planner's, in the dispatch table too or with the table left out, and says
+whether their slots are NaN (no token) and the other requests' outputs right.
+
 {"precision": [group, head_dim], "dtype": ...} gives the relative 2-norm error of the attention's
 fp32 split slots against 64 bits, before any rounding of an output.
 """
@@ -275,6 +279,34 @@ def _precision(emu, group, d, dtype):
                 records=p["record_count"], error=float((num / den) ** 0.5))
 
 
+def _spans(emu, spans, page, dispatch, group, d):
+    import numpy as np
+    import torch
+    import driver as D
+    from sglang_decode.config import DecodeConfig
+    n = len(spans) + 2
+    c = DecodeConfig(batch_capacity=n, max_splits=1, max_context=256, query_heads=2 * group, kv_heads=2, head_dim=d,
+                     page_size=page, workers=3)
+    lengths, kind = [100] * n, torch.bfloat16
+    inputs, oracle = _inputs(c, lengths, page == 1, 5, kind)
+
+    def edit(plan):
+        for i, (b, e) in enumerate(spans):
+            plan.begin[i], plan.end[i] = b, e
+        units = plan.dispatch
+        for u in range(2 * len(spans)):
+            units[u][4:6] = spans[units[u][2]] if units[u][2] < len(spans) else units[u][4:6]
+        if not dispatch:
+            units[:, 7] = 0  # no entry's kind matches: records are read from their tables
+
+    r = D.decode(emu, c, lengths, [1] * n, *inputs, mode=1, edit=edit)
+    empty, rest = r["partial"][:len(spans)], r["out"][len(spans):]
+    exact = oracle(None)[len(spans):n]
+    return dict(case="spans", kernel=r["kernel"], records=r["plan"]["record_count"],
+                empty_nan=bool(np.isnan(empty).all()),
+                violations=int((np.abs(rest - exact) > 2e-2 + 1e-2 * np.abs(exact)).sum()), nans=int(np.isnan(rest).sum()))
+
+
 def run(cases, asan):
     import torch
     import driver as D
@@ -286,6 +318,9 @@ def run(cases, asan):
         elif "upstream" in case:
             lengths, smax = case["upstream"]
             print(json.dumps(_upstream(emu, list(lengths), int(smax), getattr(torch, case.get("dtype", "bfloat16")))),
+                  flush=True)
+        elif "spans" in case:
+            print(json.dumps(_spans(emu, case["spans"], case["page"], case["dispatch"], case["group"], case["d"])),
                   flush=True)
         elif "precision" in case:
             print(json.dumps(_precision(emu, *case["precision"], getattr(torch, case["dtype"]))), flush=True)

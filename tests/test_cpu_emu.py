@@ -145,6 +145,21 @@ def test_few_workers_walk_long_task_chains(asan_build):
     _assert_clean(rc, rows, err, 10 + 1 + 1)
 
 
+def test_records_without_a_token(asan_build):
+    """Records that a caller of the C entry may hand over though the planner never emits them: begin = end at 0 (no
+    index before the table is read) and further on.  Their slots hold no value, the other requests'
+    outputs are right; with and without dispatch entries, CSR and paged."""
+    spans = [[0, 0], [64, 64], [100, 100], [0, 0]]
+    cases = [{"spans": spans, "page": p, "dispatch": t, "group": g, "d": d}
+             for p, t, g, d in ((1, True, 4, 128), (1, False, 8, 64), (16, True, 16, 256), (12, False, 1, 128))]
+    rc, rows, err = _run(cases, timeout=120)
+    assert rc == 0 and "ERROR: AddressSanitizer" not in err, err[-4000:]
+    assert len(rows) == len(cases), err[-2000:]
+    for r in rows:
+        assert r["kernel"] != "generic" and r["records"] == 6 and r["empty_nan"], r
+        assert r["violations"] == 0 and r["nans"] == 0, r
+
+
 def test_probabilities_are_held_beyond_the_kv_dtype(asan_build):
     """The fp32 split slots against 64 bits, for the groups and head dims that deal a task to fewer
     waves than eight (groups up to 4) or four (head_dim 256).  A wave's largest probability is an exact 1, so with
