@@ -498,7 +498,7 @@ __device__ __forceinline__ void tile_step(const sgd_decode_args &a, TileRegs<D> 
 template <int D>
 __device__ __forceinline__ int32_t wave_tiles(int32_t start, int32_t end, int wave) {
     constexpr int kTile = PGeo<D>::kTile, kWaves = PGeo<D>::kWaves;
-    const int32_t n = (int32_t)((uint32_t)(end - start + kTile - 1) / kTile);
+    const int32_t n = (int32_t)((uint32_t)(max(end - start, 0) + kTile - 1) / kTile);  // none for end < start
     return n > wave ? (int32_t)((uint32_t)(n - wave + kWaves - 1) / kWaves) : 0;
 }
 

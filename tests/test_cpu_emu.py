@@ -147,9 +147,10 @@ def test_few_workers_walk_long_task_chains(asan_build):
 
 def test_records_without_a_token(asan_build):
     """Records that a caller of the C entry may hand over though the planner never emits them: begin = end at 0 (no
-    index before the table is read) and further on.  Their slots hold no value, the other requests'
-    outputs are right; with and without dispatch entries, CSR and paged."""
-    spans = [[0, 0], [64, 64], [100, 100], [0, 0]]
+    index before the table is read) and further on, and end before begin (no tile is walked).  Their slots
+    hold no value, the other requests' outputs are right; with and without dispatch entries, CSR
+    and paged."""
+    spans = [[0, 0], [64, 64], [70, 10], [0, 0]]
     cases = [{"spans": spans, "page": p, "dispatch": t, "group": g, "d": d}
              for p, t, g, d in ((1, True, 4, 128), (1, False, 8, 64), (16, True, 16, 256), (12, False, 1, 128))]
     rc, rows, err = _run(cases, timeout=120)
