@@ -17,6 +17,10 @@ namespace sgd {
 namespace {
 
 constexpr int kStoreThreads = 256;
+// Workgroups of a launch, unless the batch alone is more: beyond them a token's workgroups loop over its
+// pieces (768 tokens of 64 / 8 heads: 5.6 us, 6.1 with a workgroup for every 256 pieces, 6.0 with a
+// limit of 1024; 512 tokens of 32 / 8 heads: 3.9, 4.1 with a limit of 2048).
+constexpr int kStoreGroups = 1536;
 
 struct StoreArgs {
     const char *k_new, *v_new;   // [batch, Hkv, D] (may be null: no KV write)
@@ -30,32 +34,56 @@ struct StoreArgs {
     int32_t loc64;
 };
 
-// Latency-bound (12 KB per token at the 8B shape): one 16-byte piece per thread, so that a
-// token's pieces are one round trip, made together with its slot's; with one workgroup per
-// token looping over them it was a round trip for the slot and one per 256 pieces: 1.3 us a
-// layer less in a 16-layer step of two tokens (64 / 8 heads), 0.6 at 48 tokens (32 / 8 heads).
+// Where one kind of rows (K, V or q) comes from and goes to for a token: its row in both, and the
+// stride between heads.
+struct Rows {
+    const char *src;
+    char *dst;
+    int64_t from, to;
+};
+
+// Latency-bound while the pieces fit the chip (12 KB per token at the 8B shape): one 16-byte piece per
+// thread, so that a token's pieces are one round trip, made together with its slot's.  With one
+// workgroup per token looping over them it was a round trip for the slot and one per 256 pieces (one token,
+// 32 / 8 heads: 2.7 us, now 2.3).  With thousands of tokens the address arithmetic counts: a wave
+// whose pieces are of one kind has their strides in scalar registers (1024 tokens of 32 / 8 heads:
+// 5.1 us; 5.6 with the strides loaded per lane and without the limit above; 4.9 with one workgroup
+// per token).
 __global__ __launch_bounds__(kStoreThreads) void k_store_kv_stage_q(StoreArgs a) {
     const int32_t b = blockIdx.x;
     const int32_t kv_pieces = a.k_new ? a.hkv * a.chunks : 0;
     const int32_t q_pieces = a.q_in ? a.hq * a.chunks : 0;
+    int64_t slot = -1;
+    if (kv_pieces) {
+        slot = a.loc64 ? static_cast<const int64_t *>(a.loc)[b] : static_cast<const int32_t *>(a.loc)[b];
+        if (slot >= a.cache_tokens) slot = -1;
+    }
+    const Rows k{a.k_new + b * a.kn[0], a.k_cache + slot * a.kc[0], a.kn[1], a.kc[1]};
+    const Rows v{a.v_new + b * a.vn[0], a.v_cache + slot * a.vc[0], a.vn[1], a.vc[1]};
+    const Rows q{a.q_in + b * a.qi[0], a.q_out + b * a.qo[0], a.qi[1], a.qo[1]};
     // pieces [0, kv) are K rows, [kv, 2 kv) V rows, then q rows; piece = (head, chunk)
     const int64_t pieces = 2 * (int64_t)kv_pieces + q_pieces;
     for (int64_t p = (int64_t)blockIdx.y * kStoreThreads + threadIdx.x; p < pieces;
-         p += (int64_t)gridDim.y * kStoreThreads) {  // once, unless the grid's limit cut it
-        const bool is_q = p >= 2 * (int64_t)kv_pieces, is_v = !is_q && p >= kv_pieces;
-        const int32_t r = (int32_t)(is_q ? p - 2 * (int64_t)kv_pieces : is_v ? p - kv_pieces : p);
+         p += (int64_t)gridDim.y * kStoreThreads) {
+        const int kind = p < kv_pieces ? 0 : p < 2 * (int64_t)kv_pieces ? 1 : 2;
+        const int32_t r = (int32_t)(p - kind * (int64_t)kv_pieces);
         const int32_t h = (int32_t)((uint32_t)r / (uint32_t)a.chunks), c = r - h * a.chunks;
-        const int64_t *from = is_q ? a.qi : is_v ? a.vn : a.kn, *to = is_q ? a.qo : is_v ? a.vc : a.kc;
-        const char *src = (is_q ? a.q_in : is_v ? a.v_new : a.k_new) + b * from[0] + h * from[1] + c * 16;
-        char *dst = (is_q ? a.q_out : is_v ? a.v_cache : a.k_cache) + h * to[1] + c * 16;
-        const uint4 w = *reinterpret_cast<const uint4 *>(src);
-        int64_t row = b;
-        if (kv_pieces) {
-            const int64_t slot =
-                a.loc64 ? static_cast<const int64_t *>(a.loc)[b] : static_cast<const int32_t *>(a.loc)[b];
-            if (!is_q) row = slot >= 0 && slot < a.cache_tokens ? slot : -1;
+        auto copy = [&](const Rows &x) {
+            const uint4 w = *reinterpret_cast<const uint4 *>(x.src + h * x.from + c * 16);
+            if (kind == 2 || slot >= 0) *reinterpret_cast<uint4 *>(x.dst + h * x.to + c * 16) = w;
+        };
+        const int first = __builtin_amdgcn_readfirstlane(kind);
+        if (__ballot(kind != first) != 0) {
+            auto pick = [&](auto x, auto y, auto z) { return kind == 0 ? x : kind == 1 ? y : z; };
+            copy(Rows{pick(k.src, v.src, q.src), pick(k.dst, v.dst, q.dst), pick(k.from, v.from, q.from),
+                      pick(k.to, v.to, q.to)});
+        } else if (first == 0) {
+            copy(k);
+        } else if (first == 1) {
+            copy(v);
+        } else {
+            copy(q);
         }
-        if (row >= 0) *reinterpret_cast<uint4 *>(dst + row * to[0]) = w;
     }
 }
 
@@ -117,7 +145,8 @@ extern "C" int sgd_store_kv_stage_q(const void *k_new, const void *v_new, const 
     clear_stale_error();
     const int64_t pieces = (int64_t)a.chunks * ((kv ? 2 * (int64_t)kv_heads : 0) + (q ? query_heads : 0));
     const int64_t parts = (pieces + kStoreThreads - 1) / kStoreThreads;
-    hipLaunchKernelGGL(k_store_kv_stage_q, dim3(batch, (unsigned)(parts < 65535 ? parts : 65535)), dim3(kStoreThreads), 0,
+    const int64_t most = batch < kStoreGroups ? kStoreGroups / batch : 1;
+    hipLaunchKernelGGL(k_store_kv_stage_q, dim3(batch, (unsigned)(parts < most ? parts : most)), dim3(kStoreThreads), 0,
                        (hipStream_t)stream, a);
     return launch_status("store_kv_stage_q");
 }
