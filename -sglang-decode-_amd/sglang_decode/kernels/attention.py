@@ -5,6 +5,7 @@ reference does, but passes element strides as runtime int64 arguments instead
 of compile-time constants, so a new layout never recompiles anything.
 """
 import ctypes
+import operator
 
 import torch
 
@@ -54,13 +55,22 @@ def checked_layout(config, q, k, v, pages, indptr, out_dtype=None, who="execute"
             (0, 0), True)
 
 
-def plan_args(plan):
+PLAN_FIELDS = ("lengths", "request", "split", "begin", "end", "order", "offsets", "chunk", "active",
+               "record_count", "mode", "pack_first", "pack_count", "num_packs", "static_head", "static_next")
+_plan_tensors = operator.attrgetter(*PLAN_FIELDS)
+
+
+def plan_pointers(plan):
+    """Where the plan's buffers are now, in PLAN_FIELDS order."""
+    return [t.data_ptr() for t in _plan_tensors(plan)]
+
+
+def plan_args(plan, pointers=None):
     """A sgd_decode_args with the plan's pointers and configuration; the launch's own (q, K/V,
     indices, strides, the layer's buffers) are left zero."""
     a, c = _lib.DecodeArgsC(), plan.config
-    for name in ("lengths", "request", "split", "begin", "end", "order", "offsets", "chunk", "active",
-                 "record_count", "mode", "pack_first", "pack_count", "num_packs", "static_head", "static_next"):
-        setattr(a, name, getattr(plan, name).data_ptr())
+    for name, pointer in zip(PLAN_FIELDS, plan_pointers(plan) if pointers is None else pointers):
+        setattr(a, name, pointer)
     a.query_heads, a.kv_heads, a.head_dim = c.query_heads, c.kv_heads, c.head_dim
     a.max_splits, a.page_size, a.workers = c.max_splits, c.page_size, c.workers
     return a

@@ -1,5 +1,6 @@
 """The C views a plan keeps (plan build and attention launch) follow a buffer or configuration
-that is put in another's place, and the attention's arguments take any object with a plan's fields."""
+that is put in another's place, the attention's also one whose storage is replaced in the tensor itself,
+and the attention's arguments take any object with a plan's fields."""
 import types
 
 import pytest
@@ -22,6 +23,18 @@ def test_views_follow_replaced_buffers(field):
     assert plan.decode_args().workers == 7
     lookalike = types.SimpleNamespace(**{k: v for k, v in vars(plan).items() if not k.startswith("_")})
     assert bytes(plan_args(lookalike)) == bytes(plan.decode_args())
+
+
+@pytest.mark.parametrize("field", ["lengths", "mode", "order", "static_next"])
+def test_arguments_follow_storage_replaced_in_place(field):
+    plan = PlanBuffers(DecodeConfig(batch_capacity=4, max_splits=2, max_context=256), "cpu")
+    plan.decode_args()
+    tensor = getattr(plan, field)
+    for change in (lambda: tensor.set_(tensor.clone()), lambda: setattr(tensor, "data", tensor.clone())):
+        before = tensor.data_ptr()
+        change()
+        assert tensor.data_ptr() != before and getattr(plan.decode_args(), field) == tensor.data_ptr()
+    assert bytes(plan_args(plan)) == bytes(plan.decode_args())
 
 
 def test_each_launch_has_its_own_arguments():
