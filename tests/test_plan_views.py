@@ -1,9 +1,12 @@
 """The C views a plan keeps (plan build and attention launch) follow a buffer or configuration
 that is put in another's place, the attention's also one whose storage is replaced in the tensor itself,
-and the attention's arguments take any object with a plan's fields."""
+and the attention's arguments take any object with a plan's fields.  A copied plan makes its own."""
+import copy
+import pickle
 import types
 
 import pytest
+import torch
 
 from sglang_decode.config import DecodeConfig
 from sglang_decode.kernels.attention import plan_args
@@ -35,6 +38,16 @@ def test_arguments_follow_storage_replaced_in_place(field):
         change()
         assert tensor.data_ptr() != before and getattr(plan.decode_args(), field) == tensor.data_ptr()
     assert bytes(plan_args(plan)) == bytes(plan.decode_args())
+
+
+def test_a_launched_plan_copies_and_pickles():
+    plan = PlanBuffers(DecodeConfig(batch_capacity=4, max_splits=2, max_context=256), "cpu")
+    plan.c_struct(), plan.decode_args()
+    plan.lengths.fill_(7)
+    for other in (copy.deepcopy(plan), pickle.loads(pickle.dumps(plan))):
+        assert torch.equal(other.arena, plan.arena) and other.config == plan.config
+        assert other.decode_args().lengths == other.lengths.data_ptr() != plan.lengths.data_ptr()
+        assert other.c_struct().lengths == other.lengths.data_ptr()
 
 
 def test_each_launch_has_its_own_arguments():
