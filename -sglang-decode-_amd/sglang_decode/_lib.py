@@ -115,7 +115,8 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def stream_handle(device=None):
-    if _raw_stream is not None and device is not None and device.type == "cuda" and device.index is not None:
+    if (_raw_stream is not None and isinstance(device, torch.device) and device.type == "cuda"
+            and device.index is not None):
         return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 

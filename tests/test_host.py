@@ -8,6 +8,7 @@ import re
 import types
 
 import pytest
+import torch
 
 from sglang_decode.config import DecodeConfig, Mode
 from sglang_decode.planning import reference as R
@@ -494,3 +495,12 @@ def test_plan_entries_reject_unknown_forced_modes():
         assert b"force_mode" in lib.sgd_last_error()
         assert lib.sgd_order_and_packs(None, None, None, None, None, None, None, None, 0, bad, 2, 8, 2, 64,
                                        None) == -22
+
+
+@pytest.mark.parametrize("device", [None, 0, "cuda", "cuda:0", torch.device("cuda")])
+def test_stream_handle_takes_what_current_stream_takes(device, monkeypatch):
+    """Devices without an index of their own, given as text or as a number: torch.cuda.current_stream's."""
+    from sglang_decode import _lib
+    asked = []
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: asked.append(d) or types.SimpleNamespace(cuda_stream=5))
+    assert _lib.stream_handle(device) == 5 and asked == [device]
