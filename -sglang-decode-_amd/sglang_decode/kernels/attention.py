@@ -81,7 +81,8 @@ def persistent_decode(plan, layer, q, k, v, pages, indptr, scale, k_strides, v_s
     """One attention launch.  ``write_single``: the tasks that are their request's only
     split also write their row of ``layer.output`` (contiguous [Bcap, Hq, D] in q's dtype),
     so the merge may skip those rows (kernels.merge.merge_splits with min_splits 2)."""
-    a = plan.decode_args() if hasattr(plan, "decode_args") else plan_args(plan)
+    # the class's method: an object that passes it on from a plan may have fields of its own
+    a = plan.decode_args() if hasattr(type(plan), "decode_args") else plan_args(plan)
     a.q, a.k, a.v = q.data_ptr(), k.data_ptr(), v.data_ptr()
     a.pages = pages.data_ptr()
     if indptr is not None:

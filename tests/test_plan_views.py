@@ -40,6 +40,37 @@ def test_arguments_follow_storage_replaced_in_place(field):
     assert bytes(plan_args(plan)) == bytes(plan.decode_args())
 
 
+def test_a_wrapper_keeps_the_fields_it_replaces(monkeypatch):
+    """An object that hands everything but some fields of its own on to a plan: the launch takes those fields."""
+    from sglang_decode.kernels import attention as A
+
+    class Wrapper:
+        def __init__(self, plan):
+            self.plan, self.lengths = plan, plan.lengths.clone()
+
+        def __getattr__(self, name):
+            return getattr(self.plan, name)
+
+    seen = []
+
+    class Library:
+        def sgd_persistent_decode(self, args, stream):
+            seen.append(args._obj.lengths)
+            return 0
+
+        def sgd_attention_kernel(self, args):
+            return 1
+
+    monkeypatch.setattr(A._lib, "lib", lambda: Library())
+    monkeypatch.setattr(A._lib, "stream_handle", lambda device: 0)
+    plan = PlanBuffers(DecodeConfig(batch_capacity=4, max_splits=2, max_context=256), "cpu")
+    wrapper, x = Wrapper(plan), torch.zeros((4, 32, 128), dtype=torch.bfloat16)
+    layer = types.SimpleNamespace(counter=x, partial=x, lse=x, output=x)
+    for p in (plan, wrapper):
+        A.persistent_decode(p, layer, x, x, x, x, None, 1.0, (1,) * 4, (1,) * 4, (1, 1), False)
+    assert seen == [plan.lengths.data_ptr(), wrapper.lengths.data_ptr()]
+
+
 def test_a_launched_plan_copies_and_pickles():
     plan = PlanBuffers(DecodeConfig(batch_capacity=4, max_splits=2, max_context=256), "cpu")
     plan.c_struct(), plan.decode_args()
