@@ -23,8 +23,8 @@ bool vector_layout(const sgd_decode_args &a) {
     return true;
 }
 
-// The pipelined kernel: groups up to 16 (the MFMA's N), those layouts, and page strides that
-// keep a 32-bit index times the stride a valid 64-bit byte offset.
+// The pipelined kernel: groups up to 16 (the MFMA's N), those layouts, and page strides below 2^40
+// elements (beyond any allocation; an index's byte offset is bounded by the pool it lies in).
 bool pipe_supported(const sgd_decode_args &a, int max_group) {
     const int g = a.query_heads / a.kv_heads;
     return g <= max_group && vector_layout(a) && a.k_stride[0] < (1ll << 40) && a.v_stride[0] < (1ll << 40);

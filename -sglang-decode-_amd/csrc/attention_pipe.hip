@@ -104,7 +104,6 @@ struct PGeo {
     static constexpr int kVWords = D / 32;           // 32-bit words of V per lane and slot
     static constexpr int kBlocks = D / 16;           // O^T blocks
     static constexpr int kRowDims = D == 64 ? 4 : 8; // dims per output row: row r of block b is dim kRowDims r + b
-    static constexpr int kRowChunks = D / 8;         // 16 B pieces of a K row
     static constexpr int kKLoads = kTile * D / 512;  // 16 B loads per lane for a tile's K rows
     static constexpr int kStage = kTile * 2 * D;     // bytes of a wave's K tile in LDS
     static constexpr int kQRow = 2 * D + kQPad;      // bytes of a q row in LDS
@@ -505,7 +504,7 @@ __device__ __forceinline__ int32_t wave_tiles(int32_t start, int32_t end, int wa
 // ------------------------------------------------------------------ helper wave
 // Walks the worker's units (a task in R0, R1 and STATIC, a pack in D1/D4; modes and claims as
 // in for_each_task of attention_common.h) one task ahead of the compute waves.
-template <int DT, bool CSR, int D, bool kPow2>
+template <bool CSR, int D, bool kPow2>
 __device__ __forceinline__ void helper_wave(const sgd_decode_args &a, PipeShared<D> &sh, char *sq, int32_t G, int lane,
                                             const PageMap<kPow2> &pm) {
     using GG = PGeo<D>;
@@ -654,7 +653,7 @@ __global__ __launch_bounds__(PGeo<D>::kThreads, PGeo<D>::kWavesPerSimd) void k_a
     float *const so = reinterpret_cast<float *>(sq + 2 * G * GG::kQRow);
     const PageMap<kPow2> pm(a.page_size);
     if (wave == kWaves) {
-        helper_wave<DT, CSR, D, kPow2>(a, sh, sq, G, lane0, pm);
+        helper_wave<CSR, D, kPow2>(a, sh, sq, G, lane0, pm);
         return;
     }
     const float scale2 = a.scale * kLog2e;
