@@ -120,7 +120,7 @@ def test_noncontiguous_kv_strides():
 def test_views_of_packed_projection_and_fused_kv(hq, kernel):
     """q as heads of a packed [B, (Hq + 2 Hkv) D] projection and CSR K/V as halves of one
     [tokens, 2, Hkv, D] buffer: row strides that are not Hq D / Hkv D, unit dim strides, so
-    the tuned kernels take them (sglang_backend.py:102-103 hands the kernel such views)."""
+    the pipelined kernel takes them (sglang_backend.py:102-103 hands the kernel such views)."""
     c = DecodeConfig(batch_capacity=8, max_splits=8, max_context=2048, query_heads=hq, kv_heads=8, page_size=1,
                      workers=64)
     lengths = [1, 100, 2048, 517, 0, 64]
@@ -198,7 +198,7 @@ def test_auto_kernel_is_bitwise_repeatable_at_any_worker_count(workers):
 @pytest.mark.parametrize("mode", list(Mode))
 @pytest.mark.parametrize("hq", [8, 32, 64, 128])
 def test_mfma_kernel_groups_paged(hq, mode, dtype):
-    """Groups 1, 4, 8 (Llama-3-70B heads) and 16 on the MFMA kernel (heads padded to 16):
+    """Groups 1, 4, 8 (Llama-3-70B heads) and 16 on the pipelined kernel under "mfma":
     page 16, ragged lengths (a 1-token request, a 31-token one that ends mid-tile, an
     empty row)."""
     c = DecodeConfig(batch_capacity=6, max_splits=16, max_context=4096, query_heads=hq, kv_heads=8,
@@ -217,7 +217,7 @@ def test_mfma_kernel_csr(mode):
                      head_dim=128, page_size=1, workers=40)
     lengths = [3000, 17, 640, 1, 2049, 0, 33, 700]
     q, k, v, indptr, indices = W.make_csr_inputs(c, lengths, seed=29, pool_tokens=1 << 14)
-    engine = DecodeEngine(c, force_mode=mode)  # auto picks the MFMA kernel for group 8
+    engine = DecodeEngine(c, force_mode=mode)  # auto names it "mfma" for group 8
     out = run(engine, lengths, (q, k, v, indices), indptr=indptr)
     assert engine.attention_kernel_name() == "mfma"
     close(out[:8], OA.csr_attention(q, k, v, indptr, indices, lengths)[:8])
@@ -340,7 +340,7 @@ def test_two_engines_on_two_streams():
 @pytest.mark.parametrize("page", [3, 12, 48])
 @pytest.mark.parametrize("hq", [32, 64])
 def test_page_sizes_not_a_power_of_two(page, hq):
-    """Pages of 3, 12 and 48 tokens on the tuned kernels (tokens mapped to (page, row) by
+    """Pages of 3, 12 and 48 tokens on the pipelined kernel (tokens mapped to (page, row) by
     division) and the generic one, group 4 and 8, tasks and tiles crossing page ends."""
     c = DecodeConfig(batch_capacity=6, max_splits=8, max_context=3000, query_heads=hq, kv_heads=8, page_size=page,
                      workers=96)

@@ -2,9 +2,9 @@
 each case draws its own configuration -- GQA group 1-16, head_dim 64/128/256, paged (page
 sizes 2-64 and a non-power-of-two 12) or CSR, batch capacity, worker count, max_splits,
 ragged lengths with empty rows and rows at max_context, per-request split counts, scale,
-dtype, schedule -- and runs it on every kernel that supports the shape (the reference's
-own tests fix their shapes, tests/gpu/test_decode.py; the sweep covers the combinations
-between them).  Each case prints its draw first, so a failure names it."""
+dtype, schedule -- and runs it on both kernels, the pipelined one under the name its group goes by and the
+generic one, whose math shares nothing with it (the reference's own tests fix their shapes,
+tests/gpu/test_decode.py; the sweep covers the combinations between them).  Each case prints its draw first, so a failure names it."""
 import numpy as np
 import pytest
 import torch
@@ -51,13 +51,11 @@ def draw(seed):
 
 
 def kernels_for(c, csr):
-    """The kernels whose host checks accept the shape (csrc/attention.hip select_kernel): the
-    MFMA kernel (groups <= 16) and the VALU kernel (groups <= 4) take head_dim 64, 128 and 256
-    and any page size (a power of two by shift and mask, any other by division)."""
-    ks = ["generic", "mfma"]
-    if c.group_size <= 4:
-        ks.append("valu")
-    return ks
+    """The kernels that accept the shape (csrc/attention.hip resolve_kernel): the generic one and the
+    pipelined one, "valu" for groups <= 4 and "mfma" for 8 and 16 ("mfma" for a small group runs
+    the very same build).  It takes head_dim 64, 128 and 256 and any page size (a power of two
+    by shift and mask, any other by division)."""
+    return ["generic", "valu" if c.group_size <= 4 else "mfma"]
 
 
 @pytest.mark.parametrize("seed", range(CASES))

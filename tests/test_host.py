@@ -248,7 +248,7 @@ def test_attention_kernel_selection_is_host_only():
     for workers in (108, 256, 512):
         args.workers = workers
         assert _lib.KERNEL_NAMES[lib.sgd_attention_kernel(ctypes.byref(args))] == "valu"
-    # paged with a page size that is not a power of two: still the tuned kernels
+    # paged with a page size that is not a power of two: still the pipelined kernel
     args.csr, args.page_size = 0, 12
     args.k_stride[:] = [12 * 1024, 1024, 128, 1]
     args.v_stride[:] = [12 * 1024, 1024, 128, 1]
@@ -259,14 +259,14 @@ def test_attention_kernel_selection_is_host_only():
     args.csr, args.page_size = 1, 1
     args.k_stride[:] = [1024, 0, 128, 1]
     args.v_stride[:] = [1024, 0, 128, 1]
-    args.query_heads = 64  # group 8: no VALU kernel, the MFMA one serves it
+    args.query_heads = 64  # group 8: goes by "mfma"
     assert _lib.KERNEL_NAMES[lib.sgd_attention_kernel(ctypes.byref(args))] == "mfma"
     args.kernel = _lib.KERNELS["valu"]
     assert lib.sgd_attention_kernel(ctypes.byref(args)) == -22
     assert b"group <= 4" in lib.sgd_last_error()
     args.kernel = _lib.KERNELS["mfma"]
     assert _lib.KERNEL_NAMES[lib.sgd_attention_kernel(ctypes.byref(args))] == "mfma"
-    for d in (64, 256):  # group 8: the MFMA kernel at every head dim
+    for d in (64, 256):  # group 8: "mfma" at every head dim
         args.head_dim = d
         args.k_stride[:] = [8 * d, 0, d, 1]
         args.v_stride[:] = [8 * d, 0, d, 1]
@@ -280,7 +280,7 @@ def test_attention_kernel_selection_is_host_only():
     assert lib.sgd_attention_kernel(ctypes.byref(args)) == -22
     args.kernel = _lib.KERNELS["auto"]
     assert _lib.KERNEL_NAMES[lib.sgd_attention_kernel(ctypes.byref(args))] == "generic"
-    args.query_heads = 32  # group 4: the VALU kernel at every head_dim
+    args.query_heads = 32  # group 4: "valu" at every head_dim
     for d in (64, 128, 256):
         args.head_dim = d
         args.k_stride[:] = [8 * d, 0, d, 1]
