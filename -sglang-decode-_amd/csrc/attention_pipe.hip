@@ -556,9 +556,10 @@ __device__ __forceinline__ void helper_wave(const sgd_decode_args &a, PipeShared
                                                                        : uni(a.indptr[info.request]);
             const int32_t *rows = CSR ? a.pages + ind0 : a.pages + (int64_t)info.request * a.pt_stride[0];
             // A record without a token has no last one to repeat (end - 1 may lie before the table), and
-            // nothing uses its indices: it reads a word that is there.  (A branch cost up to 47 SGPR spills.)
+            // nothing uses its indices: it reads its request's first page, or kv_indptr's first word.  (A
+            // branch spills up to 47 SGPRs more, another word's pointer 37: 0.6 us a launch of one request.)
             const bool some = info.end > info.start;
-            rows = some ? rows : a.mode;
+            if constexpr (CSR) rows = some ? rows : a.indptr;
             const int32_t last = some ? info.end - 1 : 0;
             constexpr int kIdx = GG::kTile * GG::kWaves, kLoads = (kIdx + 63) / 64;
             int32_t tile_idx[kLoads];
