@@ -2,14 +2,15 @@
 // stride -- the pipelined MFMA kernel.
 //
 // What bounds it: the K/V rows are read once, so the chip's rate of scattered 256 B row reads
-// does (6.1 TB/s measured for a plain gather of a 64-request 8B-class layer's rows, 6.4 with the
-// rows of one head after the other, 6.6 streaming the same bytes) -- as long as enough of them are in
-// flight.  A worker that stops loading at a task's end (merge barrier, then claim ->
+// does (6.1 TB/s measured for a plain gather of the 395 MB of a 64-request 8B-class layer's rows, 6.4
+// with the rows of one head after the other, 6.6 streaming as many bytes in one launch) -- as long as
+// enough of them are in flight.  A worker that stops loading at a task's end (merge barrier, then claim ->
 // record -> indices -> rows, a round trip each) leaves its share unused, and so does a wave
 // whose tile math takes as long as the rows' round trip.  Hence:
 //
 // * The math runs on the matrix cores, also for small groups: a 16 KB tile takes 16 (group <= 16)
-//   MFMAs and ~300 VALU instructions, against ~790 for packed dot products with 4 heads.
+//   MFMAs and 325 (8 heads) to 340 (4 heads) VALU instructions, all of a launch's counted, against ~790
+//   for packed dot products with 4 heads.
 // * Loads cross task boundaries.  A helper wave beside the kWaves compute waves finds the
 //   worker's next task while the current one streams, and leaves its record, its q rows
 //   and the first tiles' indices in LDS (two slots by task parity).  A compute wave
@@ -21,11 +22,11 @@
 //   both in an eight-wave form.  So K rows pass through a wave's LDS tile; V rows are
 //   operands as they come.
 //
-// Measured (us per launch, captured graph; before = a VALU kernel for groups <= 4 and a separate MFMA
-// kernel with 64 B row pieces): 8B-class heads, 64 requests, 395 MB 74.3 -> 72; 70B-class heads, 32
-// requests in 16-token pages, 1.14 GB 193 -> 186; 32 kv heads, no grouping, 537 MB 103 -> 95; head_dim 64
-// 58.9 -> 51.5; head_dim 256 82.5 -> 78; one request of 8k tokens 18.1 -> 12.8 (15.6 with every worker counted); one kv head of 8 query heads,
-// 64 requests 24.5 -> 21.1.
+// Measured, us a layer of a captured step with its plan and merges (before = a VALU kernel for groups up
+// to 4 and a separate MFMA kernel with 64 B row pieces): 8B-class heads, 64 requests, 395 MB 81.3 -> 79.9
+// (the kernel alone 72.6); 70B-class heads, 32 requests in 16-token pages, 1.14 GB 211.7 -> 203.4; 32 kv
+// heads, no grouping, 537 MB 112.0 -> 103.5; head_dim 64 65.6 -> 58.3; head_dim 256 91.8 -> 85.8; one request
+// of 8k tokens 21.6 -> 17.0; one kv head of 8 query heads, 64 requests 28.7 -> 24.9.
 //
 // Lane l of a compute wave is (m, j) = (l % 16, l / 16).  MFMA operands of 16x16xK:
 // A[m][kj ..], B[kj ..][n = l % 16], D[4j + i][n], each lane group j holding K / 4
@@ -37,8 +38,8 @@
 //   softmax          per head, exp2 domain, fp32; the cross-lane maximum and the rescaling only in
 //                    tiles that raise some head's maximum.  (Letting scores exceed the maximum
 //                    by 2^8 first is no faster, and the largest p is then not the 1 that rounds
-//                    exactly: 2.2e-3 instead of 1.75e-3 off in bf16, 1.66e-3 of it the result's own
-//                    rounding.)  P is rounded to the KV dtype (kernels/attention.py:78), and where
+//                    exactly: 2.2e-3 instead of 1.75e-3 off in bf16 without remainders, 1.66e-3 of it
+//                    the result's own rounding.)  P is rounded to the KV dtype (kernels/attention.py:78), and where
 //                    fewer waves share a task than would keep that error down its remainder
 //                    is multiplied too (below).
 //   O^T += V^T . P^T the B operand is P as S^T left it; the A operand needs one dim of each of
@@ -48,22 +49,25 @@
 // The next tile's rows are requested into the registers this tile's free up, V after P.V.
 //
 // The remainder of P: a wave's largest p is 1 and rounds exactly, the other p of the heavy tokens do
-// not, so the fewer waves share a task the larger the error of the rounded P: against 64 bits, in bf16 before
-// the output's rounding, 4.6e-4 with eight waves (groups up to 4 in an earlier kernel), 5.8e-4 with
-// four, 6.2e-4 with three.  So groups up to 4, and head_dim 256 (three waves), multiply
+// not, so the fewer waves share a task the larger the error of the rounded P: against 64 bits, in bf16
+// before the output's rounding, 4.6e-4 with eight waves (groups up to 4 in an earlier kernel), 5.8e-4
+// with four, 6.2e-4 with three.  So groups up to 4, and head_dim 256 (three waves), multiply
 // P - round(P) in the KV dtype as well, which leaves 1e-6.  Groups up to 4 leave the MFMA's upper 8
-// columns free: column n + 8 takes the remainders of head n, at no MFMA more, and they go to merge rows of
-// their own (added in registers at the task's end: 0.6 to 1.1 us a launch more).  8 and 16 heads at D = 256, which
-// have no LDS for such rows, take a second MFMA a block into accumulators of their own.  It costs up to 2 %
-// of a layer's time for groups up to 4 (eight layers of 64 requests 640 -> 642 us, a layer of 128 of ~60 tokens 24.9 -> 25.6),
-// 1 to 7 % for the others (48 requests of ~1000 tokens, D 256: 8 heads 86.1 -> 87.0, 16 heads 60.9 -> 63.7).
+// columns free: column n + 8 takes the remainders of head n, at no MFMA more, and they go to merge rows
+// of their own (added in registers at the task's end: 0.6 to 1.1 us a launch more).  8 and 16 heads at
+// D = 256, which have no LDS for such rows, take a second MFMA a block into accumulators of their own.
+// It costs up to 2 % of a layer's time for groups up to 4 (eight layers of 64 requests 637.5 -> 638.9 us,
+// 16 of one request 269 -> 272.5; 4 % with 128 requests of ~60 tokens, 20.4 -> 21.2), 1 to 8 % for the
+// others (48 requests of ~1000 tokens, D 256: 8 heads 86.1 -> 87.6, 16 heads 60.9 -> 63.4).
 //
 // Geometry: two workgroups must be resident per CU (the default worker count), and the hardware
 // deals a workgroup's waves to the SIMDs in turn, so five waves take two slots of one SIMD:
 // 4 + 1 waves need 128 VGPRs (at 140 only every second workgroup starts), as do 7 + 1 at D = 64;
-// at D = 256, where a tile and its output are 128 registers, 3 + 1 waves have 256.  At 16 tokens a
-// tile D = 128 fits 8 + 1 waves only with spills: 75 us for the first layer above.  64-token
-// tiles at D = 64 (4 + 1 waves): 57.0 against 52.9 us.
+// at D = 256, where a tile and its output are 128 registers, 3 + 1 waves have 256.  (The paged builds of
+// 8 and 16 heads at D = 128, and those of pages that are no power of two, spill one or two VGPRs: a
+// store where a wave starts and a load in its helper, none in a loop.)  At 16 tokens a tile D = 128
+// fits 8 + 1 waves only with spills: 75 us for the first layer above.  64-token tiles at D = 64 (4 + 1
+// waves): 57.0 against 52.9 us.
 #include <float.h>
 
 #include "valu_ops.h"
@@ -77,7 +81,8 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr int kIndptrLds = 256;   // CSR: kv_indptr entries kept in LDS (rows beyond read memory)
 // Tiles of wave 0 left when the helper claims the next unit: the search takes about three tiles'
-// time.  1 / 2 / 3 / 5: 73.7 / 72.7 / 70.2 / 72.0 us (64 requests), 193 / 180 / 179 / 189 (70B class).
+// time.  1 / 2 / 3 / 5: 78.0 / 77.3 / 79.0 / 79.4 us a layer (64 requests; runs of one differ by up to 2.0),
+// 191 / 193 / 199 / 200 (70B class; by up to 5.8), the others within 1 of each other: it hardly matters.
 constexpr int kClaimLead = 3;
 constexpr int kOPad = 4;          // floats after a merge row: its 16 B stores spread over the banks
 constexpr int kQPad = 16;         // bytes after a q row: 16 heads' 16 B reads spread over the banks
@@ -93,8 +98,9 @@ struct PGeo {
     static_assert(D == 64 || D == 128 || D == 256, "head_dim 64, 128 or 256");
     static constexpr int kWaves = D == 64 ? 7 : D == 128 ? 4 : 3;  // compute waves per workgroup
     static constexpr int kThreads = 64 * (kWaves + 1);
-    // The next K rows are requested once this tile's are staged, or, where registers are short,
-    // not beside the scores and their operands but after them.
+    // The next K rows are requested once this tile's are staged, or not beside the scores and their
+    // operands but after them: at D = 128 for want of registers, at D = 256, which has them, because the
+    // early request is no faster (24 requests 86.1 us a layer against 85.6, others -1 to +2 %).
     static constexpr bool kEarlyK = D == 64;
     static constexpr int kWavesPerSimd = D == 256 ? 2 : 4;
     static constexpr int kTile = D == 256 ? 16 : 32; // tokens per tile
@@ -218,9 +224,8 @@ struct TileRegs {
 };
 
 // Row and 16 B piece that lane (m, j) fetches with K load i: whole 256 B (D = 64: 128 B) rows per
-// 16 (8) lanes, four (eight) rows an instruction.  Fetching the MFMA's operand layout itself, 64 B
-// of 16 rows an instruction, moves the same bytes at 5.5 instead of 7.3 TB/s (206 -> 156 us for
-// the 1.14 GB of a 70B-class layer), so the rows pass through LDS.
+// 16 (8) lanes, four (eight) rows an instruction, and not the MFMA's operand layout itself, 64 B of 16
+// rows an instruction (at the top: 78.9 against 71.6 us), so the rows pass through LDS.
 template <int D>
 __device__ __forceinline__ int k_row(int i, int m, int j) {
     if constexpr (D == 64) return 16 * (i >> 1) + 4 * j + 2 * (i & 1) + (m >> 3);
