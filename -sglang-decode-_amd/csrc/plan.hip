@@ -528,8 +528,11 @@ __device__ void stage_greedy_lists(const int32_t *weight, int32_t total, int32_t
 // kLdsRecords; a search of the offsets otherwise), the bucket of its weight -- where a walk
 // over 16 bucket tables, twice, and a binary search stood before: 18.8 -> 11.8 us a build for 4100
 // tasks, 13.7 -> 9.7 for 1776 (launch included).
+// One loop for each source of the records (kRecs): chosen per task, R1 builds of more records were
+// slower than before `recs` (65536 tasks of 4096 records 81.8 -> 85.5 us a build; 82.2 now).
 constexpr int kLdsRecords = 2048;
 
+template <bool kRecs>
 __device__ void stage_units(int32_t *table, int32_t capacity, int32_t *pack_first, int32_t *pack_count,
                             const int16_t *order_mirror, const int4 *recs, const RowMirror &rows, int32_t bcap,
                             int32_t total, const int32_t *weight, int32_t hkv, int32_t buckets, const PlanShared &sh) {
@@ -557,7 +560,7 @@ __device__ void stage_units(int32_t *table, int32_t capacity, int32_t *pack_firs
         }
         if (!table || unit < 0 || unit >= capacity) continue;
         int4 f;
-        if (recs) {
+        if constexpr (kRecs) {
             f = recs[rec];
         } else {
             const int32_t r = request_of(rows.offsets, bcap, rec);
@@ -672,8 +675,13 @@ __global__ __launch_bounds__(kPlanThreads) void k_build_plan(sgd_plan_buffers p,
     stage_order(L.b.weight, total, p.order, p.num_packs, p.mode, rules_lds ? sh.rules : p.rules, p.rule_count, force,
                 p.kv_heads, p.workers, p.buckets, p.batch_capacity * p.max_splits, sh, L.a.pre.order);
     lds_barrier();
-    stage_units(p.dispatch, p.batch_capacity * p.max_splits * p.kv_heads, p.pack_first, p.pack_count, L.a.pre.order,
-                recs, mirror, p.batch_capacity, total, L.b.weight, p.kv_heads, p.buckets, sh);
+    const int32_t units = p.batch_capacity * p.max_splits * p.kv_heads;
+    if (recs)
+        stage_units<true>(p.dispatch, units, p.pack_first, p.pack_count, L.a.pre.order, L.b.few.recs, mirror,
+                          p.batch_capacity, total, L.b.few.weight, p.kv_heads, p.buckets, sh);
+    else
+        stage_units<false>(p.dispatch, units, p.pack_first, p.pack_count, L.a.pre.order, nullptr, mirror,
+                           p.batch_capacity, total, L.b.weight, p.kv_heads, p.buckets, sh);
     if (run_greedy) {
         lds_barrier();
         // the LPT's worker keys and tails take region A (free by now), its keys replace the weights
